@@ -147,8 +147,7 @@ int ppf_solve_async_result(ppf_plan *plan, void *stream, ppf_stats *stats);
  * extents, the x- and y-pass variants (threads per line: one radix-R
  * butterfly per thread per stage, or half the threads with two) and the
  * z-pass kernel shapes (partitioned Thomas with K rows per thread and S
- * columns per workgroup, pipelined wavefront cyclic reduction); keeps the
- * fastest of each pass for later solves and returns the z shape's id in
+ * columns per workgroup); keeps the fastest of each pass for later solves and returns the z shape's id in
  * *zvariant (may be NULL).  Results are cached per problem shape (extents,
  * boundary conditions, precision) for the life of the process: a second plan
  * of a tuned shape is set without timing.  p is overwritten.  Synchronises
@@ -159,7 +158,7 @@ int ppf_plan_tune(ppf_plan *plan, const double *prhs, double *p, const double *d
                   const double *dmx3, const double *dx3, void *stream, int *zvariant);
 
 /* Pins the z-pass kernel shape (an id returned by ppf_plan_tune, 1..17; 0 =
- * the default chosen by n3m).  A shape that does not fit the plan's z extent
+ * the default chosen by the extents).  A shape that does not fit the plan's z extent
  * makes later solves return PPF_ERR_UNSUPPORTED. */
 int ppf_plan_set_zvariant(ppf_plan *plan, int zvariant);
 

@@ -8,9 +8,9 @@
 
 namespace ppf {
 
-// z row coefficients for one solve as a table (read by the residual forms and
-// the pipelined z kernel): zam[k], zap[k] (k < n3m), then zap[n3m..n3m+3] =
-// the wall extrapolation coefficients.
+// z row coefficients for one solve as a table (read by the residual forms):
+// zam[k], zap[k] (k < n3m), then zap[n3m..n3m+3] = the wall extrapolation
+// coefficients.
 static __global__ void __launch_bounds__(256)
 k_zcoef(const double *__restrict__ dx3, const double *__restrict__ dmx3, int n3m, double *__restrict__ zam,
         double *__restrict__ zap) {

@@ -1105,19 +1105,41 @@ __device__ __forceinline__ double frcp(double x) {
 // is what lets one workgroup's loads overlap another's arithmetic here).
 // CT: arithmetic type (FP64 for every plan: FP32 arithmetic on FP32 storage
 // measured no faster and costs the refinement a sweep).
+//
+// Registers bound this kernel: 2K values a thread are the algorithm's own, and
+// what it holds beside them decides how many workgroups share a CU.  Row
+// addresses are therefore formed from one base at each access, masks are
+// comparisons with one row count, a row's coefficients are one 16-byte LDS
+// read, and every step of a sweep is pinned in its place: the empty volatile
+// asm of zp_pin takes the step's state and the LDS index, so neither is the
+// arithmetic moved behind the reads of all the later steps (the compiler
+// otherwise reads the coefficients of the whole sweep first) nor are the
+// coefficients and addresses of one sweep carried to the next.
+__device__ __forceinline__ void zp_pin(int &i) { asm volatile("" : "+v"(i)); }
+__device__ __forceinline__ void zp_pin(int &i, double &a) { asm volatile("" : "+v"(i), "+v"(a)); }
+__device__ __forceinline__ void zp_pin(int &i, double &a, double &b) { asm volatile("" : "+v"(i), "+v"(a), "+v"(b)); }
+// LDS row of partition p: K coefficient pairs and one pad pair, so that the
+// partitions of a wave start on different banks
+template <int K>
+__host__ __device__ constexpr int zp_coef_slots(int rows) { return rows + rows / K + 1; }
+template <int K, int S>
+constexpr size_t zp_lds_bytes(int P) {
+    constexpr int KS = (K + S - 1) / S;  // table rows staged per thread
+    return 16 * (size_t)zp_coef_slots<K>(KS * S * P) + 7 * sizeof(double) * (size_t)P * S;
+}
 template <typename T, int K, int S, int NTMAX, int WPE, typename CT = double>
 __global__ void __launch_bounds__(NTMAX) __attribute__((amdgpu_waves_per_eu(WPE)))
 k_zpart(T *__restrict__ W, ZArgs z, const double *__restrict__ zam, const double *__restrict__ zap,
         double *__restrict__ mean_out, int P) {
     if (gated_off(z.gate)) return;
+    using D2 = double __attribute__((ext_vector_type(2)));
     extern __shared__ double zsh[];
     const int n3m = z.n3m;
     constexpr int KS = (K + S - 1) / S;           // table rows per thread
-    const int NPAD = KS * (int)blockDim.x;        // >= NP: every thread writes KS entries
-    double *am = zsh;               // [NPAD], 0 past n3m
-    double *ap = am + NPAD;         // [NPAD], 0 past n3m
+    const int NPAD = KS * (int)blockDim.x;        // >= P * K: every thread writes KS entries
+    D2 *co = reinterpret_cast<D2 *>(zsh);         // (am, ap) of row g at g + g / K; zero past n3m
     const int PS = P * S;
-    CT *ra = reinterpret_cast<CT *>(ap + NPAD);  // [3][P][S]: first-row equations, then reduction buffer
+    CT *ra = reinterpret_cast<CT *>(co + zp_coef_slots<K>(NPAD));  // [3][P][S]: first-row equations, then reduction buffer
     CT *rc = ra + 3 * PS;           // [3][P][S]: reduction buffer
     CT *xe = rc + 3 * PS;           // [P][S]: partition end values x_{K-1}
     CT *ps = ra;                    // [P][S]: partial sums, once the reduction is done
@@ -1130,15 +1152,21 @@ k_zpart(T *__restrict__ W, ZArgs z, const double *__restrict__ zam, const double
     const int kx = ct * S + s;
     const bool active = kx < z.Lx;
     const size_t pstride = (size_t)z.Ly * z.Lxs;
-    // columns past Lx (the last tile's padding) load the last real column,
-    // which lies in the same 128-byte rows, and are masked below
-    T *w = W + w_at<T>(jp, active ? kx : z.Lx - 1, z.Ly);
-    const CT lx = active ? (CT)z.lamx[kx] : CT(0);
-    const CT ly = (CT)z.lamy[jp];
-    const bool pin = active && z.zx[kx] && z.zy[jp];
     const int g0 = p * K;
-    // loads are clamped in bounds and selected, so the sweep code is branch-free
     const int glast = n3m - 1;
+    // columns past Lx (the last tile's padding) load the last real column,
+    // which lies in the same 128-byte rows, and are masked below; rows past
+    // n3m load the last row
+    const int kc0 = active ? kx : z.Lx - 1;
+    T *wl = W + w_at<T>(jp, kc0, z.Ly) + (size_t)((g0 < glast ? g0 : glast) + 1) * pstride;  // the partition's first row
+    const int lcap = glast > g0 ? glast - g0 : 0;                   // its last row to load
+    int rbytes = (int)(pstride * sizeof(T));  // bytes from row to row (a plane, below 16 MB)
+    auto row = [&](int l) -> T * {
+        return reinterpret_cast<T *>(reinterpret_cast<char *>(wl) + (size_t)(unsigned)l * (unsigned)rbytes);
+    };
+    const CT lx = (CT)z.lamx[kc0], ly = (CT)z.lamy[jp];
+    const int pin0 = (active & (z.zx[kc0] != 0) & (z.zy[jp] != 0) & (p == 0)) ? 0 : -1;  // row pinned in this partition
+    int nv = active ? n3m - g0 : 0;  // rows l < nv are real
     // Row coefficients (the per-solve table filled by pass 1) are loaded
     // first: loads complete in order, so waiting for them does not wait for
     // the line loads issued after them.  Their LDS writes are unconditional
@@ -1151,71 +1179,69 @@ k_zpart(T *__restrict__ W, ZArgs z, const double *__restrict__ zam, const double
         ca[j] = zam[kc];
         cp[j] = zap[kc];
     }
-    double bcd[4];  // z wall extrapolation, from the same table
-#pragma unroll
-    for (int q = 0; q < 4; ++q) bcd[q] = zap[n3m + q];
     // line loads in the order the two sweeps below consume them (rows 1 and
     // K-2 first, then inwards; rows 0 and K-1 last), so the sweeps start as
     // soon as the first rows arrive; nothing consumes them before that
-    CT d[K];
+    T raw[K];
 #pragma unroll
     for (int q = 0; q < K; ++q) {
         const int l = q < K - 2 ? ((q & 1) ? K - 2 - q / 2 : 1 + q / 2) : (q == K - 2 ? 0 : K - 1);
-        const int g = g0 + l;
-        d[l] = (CT)ld_stream(&w[(size_t)((g < glast ? g : glast) + 1) * pstride]);
+        raw[l] = ld_stream(row(l < lcap ? l : lcap));
     }
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
         const int k = tid + j * (int)blockDim.x;
-        am[k] = k < n3m ? ca[j] : 0.0;
-        ap[k] = k < n3m ? cp[j] : 0.0;
+        co[k + k / K] = k < n3m ? D2{ca[j], cp[j]} : D2{0.0, 0.0};
     }
-    CT bc[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) bc[q] = (CT)bcd[q];
     __syncthreads();
     // a row's value is masked where it is first used: zero past n3m, in
     // inactive columns, and in the pinned first row of the (0,0) mode
-    auto dmask = [&](int l) {
-        const int g = g0 + l;
-        d[l] = (active && g < n3m && !(pin && g == 0)) ? d[l] : CT(0);
-    };
+    CT d[K];
+    auto dmask = [&](int l) { d[l] = (l < nv && l != pin0) ? (CT)raw[l] : CT(0); };
     // identity rows: padding past n3m, and the pinned first row of the (0,0) mode
-    auto coef = [&](int l, CT &a, CT &b, CT &c) {
-        const int g = g0 + l;
-        const bool id = (g >= n3m) || (pin && g == 0);
-        const CT am_ = (CT)am[g], ap_ = (CT)ap[g];
-        a = am_;
-        c = id ? CT(0) : ap_;
-        b = id ? CT(1) : (-am_ - ap_ - lx) - ly;
+    int co0 = p * (K + 1);
+    auto coef = [&](int l, D2 ac, CT &a, CT &b, CT &c) {
+        const bool id = l >= nv || l == pin0;
+        a = (CT)ac.x;
+        c = id ? CT(0) : (CT)ac.y;
+        b = id ? CT(1) : (-(CT)ac.x - (CT)ac.y - lx) - ly;
     };
     // Reverse sweep (first-row equation) and forward sweep (last-row
     // equation) interleaved: two independent dependency chains per step.
-    // The forward pivots r_l are kept for the final pass.
+    // The forward pivots r_l are kept for the final pass.  A step reads the
+    // next one's coefficients before its own arithmetic, so the LDS latency is
+    // not in the chain.
     CT rr[K];
     CT ah, ch, dh, Af, Df, Cf;
     {
         CT a, b, c;
         dmask(K - 2);
         dmask(1);
-        coef(K - 2, a, b, c);
-        double r = frcp(b);
+        coef(K - 2, co[co0 + K - 2], a, b, c);
+        CT r = frcp(b);
         ah = r * a; ch = r * c; dh = r * d[K - 2];
-        coef(1, a, b, c);
+        coef(1, co[co0 + 1], a, b, c);
         r = frcp(b);
         rr[1] = r;
         Af = r * a; Cf = r * c; Df = r * d[1];
+        D2 nb = co[co0 + K - 3], nf = co[co0 + 2];
 #pragma unroll
         for (int i = 1; i <= K - 2; ++i) {
             const int lb = K - 2 - i;  // reverse row
             const int lf = 1 + i;      // forward row
-            dmask(lb);
-            dmask(lf);
+            const D2 cb = nb, cf = nf;
+            if (i < K - 2) {
+                nb = co[co0 + lb - 1];
+                nf = co[co0 + lf + 1];
+            }
+            // a row is masked by the sweep that meets it first
+            if (2 * lb > K - 1 || lb == 0) dmask(lb);
+            if (2 * lf < K - 1 || lf == K - 1) dmask(lf);
             CT a1, b1, c1, a2, b2, c2;
-            coef(lb, a1, b1, c1);
-            coef(lf, a2, b2, c2);
-            const double r1 = frcp(b1 - c1 * ah);
-            const double r2 = frcp(b2 - a2 * Cf);
+            coef(lb, cb, a1, b1, c1);
+            coef(lf, cf, a2, b2, c2);
+            const CT r1 = frcp(b1 - c1 * ah);
+            const CT r2 = frcp(b2 - a2 * Cf);
             ch = -r1 * c1 * ch;
             dh = r1 * (d[lb] - c1 * dh);
             ah = r1 * a1;
@@ -1223,8 +1249,8 @@ k_zpart(T *__restrict__ W, ZArgs z, const double *__restrict__ zam, const double
             Af = -r2 * a2 * Af;
             Cf = r2 * c2;
             Df = r2 * (d[lf] - a2 * Df);
-            // keep coefficient reads next to their use (register pressure)
-            __builtin_amdgcn_sched_barrier(0);
+            zp_pin(co0, dh, Df);
+            zp_pin(nv, ch, Af);
         }
     }
     // Reduced system in the partition end values e_p = x_{K-1} of partition p.
@@ -1288,56 +1314,59 @@ k_zpart(T *__restrict__ W, ZArgs z, const double *__restrict__ zam, const double
     CT *x = d;
     {
         CT e = x0;
+        CT na = (CT)co[co0 + 1].x;
 #pragma unroll
         for (int l = 1; l <= K - 2; ++l) {
-            CT a, b, c;
-            coef(l, a, b, c);
+            const CT a = na;
+            na = (CT)co[co0 + l + 1].x;
             e = rr[l] * (d[l] - a * e);
             d[l] = e;
-            __builtin_amdgcn_sched_barrier(0);
+            zp_pin(co0, e);
         }
+        zp_pin(nv);
         x[0] = x0;
         x[K - 1] = xl;
+        CT nc = (CT)co[co0 + K - 2].y;
 #pragma unroll
         for (int l = K - 2; l >= 1; --l) {
-            CT a, b, c;
-            coef(l, a, b, c);
+            const CT c = (l >= nv || l == pin0) ? CT(0) : nc;
+            nc = (CT)co[co0 + l - 1].y;
             x[l] = d[l] - rr[l] * c * x[l + 1];
-            __builtin_amdgcn_sched_barrier(0);
+            zp_pin(co0, x[l]);
+            zp_pin(nv);
         }
     }
-    double part = 0.0;  // mean: FP64 (only the (0,0) tile's sum is used)
+    asm volatile("" : "+s"(rbytes));
+    zp_pin(nv);
+    CT xt = 0, xb = 0;  // the line's last two rows, in the partition that ends it (l = nv - 1)
 #pragma unroll
     for (int l = 0; l < K; ++l) {
-        const int g = g0 + l;
-        if (g < n3m) {
-            part += x[l];
-            if (active) st_stream(&w[(size_t)(g + 1) * pstride], (T)x[l]);
-        }
+        if (l < nv) st_stream(row(l), (T)x[l]);
+        xt = l == nv - 1 ? x[l] : xt;
+        xb = l == nv - 2 ? x[l] : xb;
     }
     // spectral z ghost planes: wall extrapolation (fft_3d_poisson.f90:809-852)
     // or, for periodic z, the wrapped end planes (:666-796)
     if (active) {
-        const int gt = n3m - 1, pt = gt / K, lt = gt - pt * K;
+        const double *bc = zap + n3m;  // z wall extrapolation, from the same table
+        T *w0 = wl - (size_t)((g0 < glast ? g0 : glast) + 1) * pstride;  // plane 0 of this column
         if (p == 0) {
-            if (z.zper) w[(size_t)(n3m + 1) * pstride] = (T)x[0];
-            else w[0] = (T)(bc[0] * x[0] - bc[1] * x[1]);
+            if (z.zper) w0[(size_t)(n3m + 1) * pstride] = (T)x[0];
+            else w0[0] = (T)((CT)bc[0] * x[0] - (CT)bc[1] * x[1]);
         }
-        if (p == pt) {
-            CT xt = 0, xb = 0;
-#pragma unroll
-            for (int l = 0; l < K; ++l) {
-                if (l == lt) xt = x[l];
-                if (l == lt - 1) xb = x[l];
-            }
-            if (lt == 0) xb = xe[(pt - 1) * S + s];
-            if (z.zper) w[0] = (T)xt;
-            else w[(size_t)(n3m + 1) * pstride] = (T)(bc[2] * xt - bc[3] * xb);
+        if (nv >= 1 && nv <= K) {
+            if (nv == 1) xb = xe[(p - 1) * S + s];
+            if (z.zper) w0[0] = (T)xt;
+            else w0[(size_t)(n3m + 1) * pstride] = (T)((CT)bc[2] * xt - (CT)bc[3] * xb);
         }
     }
     // mean of the solution from the (0,0) real column (:628-664)
     const bool mean_tile = (jp == z.mean_jp) && ct * S <= z.mean_kx && z.mean_kx < ct * S + S;
     if (mean_tile) {
+        double part = 0.0;  // FP64
+#pragma unroll
+        for (int l = 0; l < K; ++l)
+            if (l < nv) part += x[l];
         ps[p * S + s] = part;
         __syncthreads();
         if (p == 0 && kx == z.mean_kx) {
@@ -1345,222 +1374,6 @@ k_zpart(T *__restrict__ W, ZArgs z, const double *__restrict__ zam, const double
             for (int q = 0; q < P; ++q) sum += ps[q * S + s];
             *mean_out = sum * z.mean_scale;
         }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// pass 3, pipelined form (an alternative shape; the default is k_zpart with
-// K = 32, S = 16, which measured faster at 512^3 on MI355X).
-//
-// Same partitioned Thomas as k_zpart, with two changes that matter on
-// gfx950:
-//  - persistent workgroups walk column tiles and prefetch the next tile's K
-//    values per thread into registers before solving the current tile, so
-//    HBM traffic overlaps the arithmetic instead of every resident
-//    workgroup loading, then computing, in lockstep;
-//  - the 2P-row reduced system of each column is transposed once through LDS
-//    so that one wavefront owns a whole column (lane i = reduced row i) and
-//    cyclic reduction runs with cross-lane shuffles: two barriers per tile.
-// ---------------------------------------------------------------------------
-template <typename T, int K, int S, int WPE>
-__global__ void __launch_bounds__(S * 32) __attribute__((amdgpu_waves_per_eu(WPE)))
-k_zpipe(T *__restrict__ W, ZArgs z, const double *__restrict__ zam, const double *__restrict__ zap,
-        double *__restrict__ mean_out, int P) {
-    if (gated_off(z.gate)) return;
-    constexpr int RS = 65;  // LDS column stride of the reduced system (2P <= 64, padded)
-    extern __shared__ double zsh[];
-    const int n3m = z.n3m;
-    const int NP = P * K;
-    const int R = 2 * P;
-    double *am = zsh;
-    double *ap = am + NP;
-    double *red_l = ap + NP;       // [S][RS]
-    double *red_u = red_l + S * RS;
-    double *red_d = red_u + S * RS;
-    double *ps = red_d + S * RS;   // [P][S] partial sums
-    const int tid = threadIdx.x, s = tid % S, p = tid / S;
-    // A column's reduced system goes to one wavefront, lane i holding row i,
-    // so only waves with at least R lanes take columns: every full wave, and
-    // the last (partial) wave only if it still has R lanes.  R = 2P <= S P, so
-    // wave 0 always qualifies.
-    const int lane = tid & 63, wv = tid >> 6;
-    const int nwv = (int)(blockDim.x >> 6) + ((int)(blockDim.x & 63) >= 2 * P ? 1 : 0);
-    for (int k = tid; k < NP; k += blockDim.x) {
-        am[k] = k < n3m ? zam[k] : 0.0;
-        ap[k] = k < n3m ? zap[k] : 0.0;
-    }
-    double bc[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) bc[q] = zap[n3m + q];
-    const int tiles_x = (z.Lx + S - 1) / S;
-    const int ntiles = tiles_x * z.njr;
-    const size_t pstride = (size_t)z.Ly * z.Lxs;
-    const int g0 = p * K;
-    const int glast = n3m - 1;
-    // Prefetch loads go to clamped, always valid addresses and nothing consumes
-    // them until the next tile starts: a select on a loaded value right after
-    // the load would make every load a full round trip (s_waitcnt per row).
-    T pre[K];
-    double pre_lx, pre_ly;
-    unsigned char pre_zx, pre_zy;
-    auto fetch = [&](int tile) {
-        const int jp = z.jlo + tile % z.njr;  // rows fastest inside a column tile
-        int kx = (tile / z.njr) * S + s;
-        kx = kx < z.Lx ? kx : z.Lx - 1;
-        const T *w = W + w_at<T>(jp, kx, z.Ly);
-#pragma unroll
-        for (int l = 0; l < K; ++l) {
-            const int g = g0 + l;
-            pre[l] = w[(size_t)((g < glast ? g : glast) + 1) * pstride];
-        }
-        pre_lx = z.lamx[kx];
-        pre_ly = z.lamy[jp];
-        pre_zx = z.zx[kx];
-        pre_zy = z.zy[jp];
-    };
-    int tile = blockIdx.x;
-    if (tile < ntiles) fetch(tile);
-    __syncthreads();
-    for (; tile < ntiles; tile += gridDim.x) {
-        const int jp = z.jlo + tile % z.njr;
-        const int kx = (tile / z.njr) * S + s;
-        const bool active = kx < z.Lx;
-        T *w = W + w_at<T>(jp, active ? kx : 0, z.Ly);
-        const double lx = active ? pre_lx : 0.0;
-        const double ly = pre_ly;
-        const bool pin = active && pre_zx && pre_zy;
-        double d[K];
-#pragma unroll
-        for (int l = 0; l < K; ++l) d[l] = (active && g0 + l < n3m) ? (double)pre[l] : 0.0;
-        if (pin && g0 == 0) d[0] = 0.0;
-        if (tile + (int)gridDim.x < ntiles) fetch(tile + gridDim.x);
-        auto coef = [&](int l, double &a, double &b, double &c) {
-            const int g = g0 + l;
-            const bool id = (g >= n3m) || (pin && g == 0);
-            const double am_ = am[g], ap_ = ap[g];
-            a = am_;
-            c = id ? 0.0 : ap_;
-            b = id ? 1.0 : (-am_ - ap_ - lx) - ly;
-        };
-        double rr[K];
-        double ah, ch, dh, Af, Df, Cf;
-        {
-            double a, b, c;
-            coef(K - 2, a, b, c);
-            double r = frcp(b);
-            ah = r * a; ch = r * c; dh = r * d[K - 2];
-            coef(1, a, b, c);
-            r = frcp(b);
-            rr[1] = r;
-            Af = r * a; Cf = r * c; Df = r * d[1];
-#pragma unroll
-            for (int i = 1; i <= K - 2; ++i) {
-                const int lb = K - 2 - i, lf = 1 + i;
-                double a1, b1, c1, a2, b2, c2;
-                coef(lb, a1, b1, c1);
-                coef(lf, a2, b2, c2);
-                const double r1 = frcp(b1 - c1 * ah);
-                const double r2 = frcp(b2 - a2 * Cf);
-                ch = -r1 * c1 * ch;
-                dh = r1 * (d[lb] - c1 * dh);
-                ah = r1 * a1;
-                rr[lf] = r2;
-                Af = -r2 * a2 * Af;
-                Cf = r2 * c2;
-                Df = r2 * (d[lf] - a2 * Df);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        red_l[s * RS + 2 * p] = ah;
-        red_u[s * RS + 2 * p] = ch;
-        red_d[s * RS + 2 * p] = dh;
-        red_l[s * RS + 2 * p + 1] = Af;
-        red_u[s * RS + 2 * p + 1] = Cf;
-        red_d[s * RS + 2 * p + 1] = Df;
-        __syncthreads();
-        // cyclic reduction of each column's reduced system inside one wavefront
-        // (waves past nwv take none; a shuffle source past R is masked below)
-        for (int col = wv; wv < nwv && col < S; col += nwv) {
-            const bool in = lane < R;
-            double l_ = in ? red_l[col * RS + lane] : 0.0;
-            double u_ = in ? red_u[col * RS + lane] : 0.0;
-            double d_ = in ? red_d[col * RS + lane] : 0.0;
-            double b_ = 1.0;
-            for (int h = 1; h < R; h <<= 1) {
-                const int im = lane - h, ip = lane + h;
-                const double lm = __shfl(l_, im < 0 ? 0 : im), bm = __shfl(b_, im < 0 ? 0 : im);
-                const double um = __shfl(u_, im < 0 ? 0 : im), dm = __shfl(d_, im < 0 ? 0 : im);
-                const double lp = __shfl(l_, ip > 63 ? 63 : ip), bp = __shfl(b_, ip > 63 ? 63 : ip);
-                const double up = __shfl(u_, ip > 63 ? 63 : ip), dp = __shfl(d_, ip > 63 ? 63 : ip);
-                const bool hm = im >= 0, hp = ip < R;
-                const double al = hm ? -l_ * frcp(bm) : 0.0;
-                const double ga = hp ? -u_ * frcp(bp) : 0.0;
-                const double nb = b_ + al * (hm ? um : 0.0) + ga * (hp ? lp : 0.0);
-                const double nl = al * (hm ? lm : 0.0);
-                const double nu = ga * (hp ? up : 0.0);
-                const double nd = d_ + al * (hm ? dm : 0.0) + ga * (hp ? dp : 0.0);
-                b_ = nb; l_ = nl; u_ = nu; d_ = nd;
-            }
-            if (in) red_d[col * RS + lane] = d_ * frcp(b_);
-        }
-        __syncthreads();
-        const double x0 = red_d[s * RS + 2 * p];
-        const double xl = red_d[s * RS + 2 * p + 1];
-        double *x = d;
-        {
-            double e = x0;
-#pragma unroll
-            for (int l = 1; l <= K - 2; ++l) {
-                double a, b, c;
-                coef(l, a, b, c);
-                e = rr[l] * (d[l] - a * e);
-                d[l] = e;
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            x[0] = x0;
-            x[K - 1] = xl;
-#pragma unroll
-            for (int l = K - 2; l >= 1; --l) {
-                double a, b, c;
-                coef(l, a, b, c);
-                x[l] = d[l] - rr[l] * c * x[l + 1];
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        double part = 0.0;
-#pragma unroll
-        for (int l = 0; l < K; ++l) {
-            const int g = g0 + l;
-            if (g < n3m) {
-                part += x[l];
-                if (active) st_stream(&w[(size_t)(g + 1) * pstride], (T)x[l]);
-            }
-        }
-        if (active) {
-            if (p == 0) w[0] = (T)(bc[0] * x[0] - bc[1] * x[1]);
-            const int gt = n3m - 1, pt = gt / K, lt = gt - pt * K;
-            if (p == pt) {
-                double xt = 0.0, xb = 0.0;
-#pragma unroll
-                for (int l = 0; l < K; ++l) {
-                    if (l == lt) xt = x[l];
-                    if (l == lt - 1) xb = x[l];
-                }
-                if (lt == 0) xb = red_d[s * RS + 2 * (pt - 1) + 1];
-                w[(size_t)(n3m + 1) * pstride] = (T)(bc[2] * xt - bc[3] * xb);
-            }
-        }
-        const int kx0 = (tile / z.njr) * S;
-        if (jp == z.mean_jp && kx0 <= z.mean_kx && z.mean_kx < kx0 + S) {
-            ps[p * S + s] = part;
-            __syncthreads();
-            if (p == 0 && kx == z.mean_kx) {
-                double sum = 0.0;
-                for (int q = 0; q < P; ++q) sum += ps[q * S + s];
-                *mean_out = sum * z.mean_scale;
-            }
-        }
-        __syncthreads();  // red_* is rewritten by the next tile
     }
 }
 

@@ -1,16 +1,57 @@
 // ppf_zpass.hip -- host launcher of pass 3 (the z Thomas solves) for FP64 and
-// FP32 workspaces: the z-pass shapes (partitioned register Thomas k_zpart, its
-// pipelined wavefront form k_zpipe, the one-thread-per-line k_zthomas) and the
-// choice among them.
+// FP32 workspaces: the shapes of the partitioned register Thomas k_zpart, the
+// one-thread-per-line k_zthomas, and the choice among them.
 #include <type_traits>
 
 #include "ppf_plan.hpp"
 
 namespace ppf {
 
+namespace {
+constexpr int kZLong8 = 18, kZLong4 = 19;
+// The shape of a plan that was not tuned, from the line length and the number
+// of 16-column workgroups.  z stage in us, 256 x 256 lines (65536 columns)
+// unless another grid is named, this rule's shape against the neighbours:
+//  * up to 512 rows, about 16 partitions: S P then fills whole groups of four
+//    waves, one for each SIMD (a six-wave workgroup of 28 or 32 rows gets one
+//    place where two would fit): 300 rows K=20 104, K=32 111, K=16 124;
+//    384 rows K=24 117, 32 122, 16 135; 448 rows K=28 127, 32 137, 16 145;
+//    200 rows K=20 66, K=16 69, K=32 73;
+//  * 513..768 rows K = 24, whose 128 registers admit two 512-thread
+//    workgroups per CU: 768 rows 266, K=28 319, K=32 348 (1024 x 1024 x 768:
+//    2.92 ms, K=32 4.31 ms);
+//  * FP32 workspaces up to 256 rows take 32 columns, whole 128-byte rows:
+//    256 rows (32,32) 46, (16,16) 59; 128 rows (16,32) 26, (8,16) 29;
+//  * fewer workgroups than four per CU (they are all resident at once, so a
+//    line's chain of rows is what counts): 8 columns and short partitions.
+//    64 x 64 lines (PP) of 64 rows: (8,8) 8.4, (16,16) 10.0, (32,16) 13.1; of
+//    512 rows (16,8) 16.1, (8,8) 18.9, (32,16) 19.6; of 768 rows (24,8) 20.8,
+//    (24,16) 25.8; of 1024 rows (32,8) 26.0, (32,16) 39.7;
+//  * over 1024 rows 8 columns (a 16-column workgroup exceeds 512 threads or
+//    its registers) and K = 48; 1537..2048 rows K = 32.  128 x 128 lines of
+//    1536 rows K=48 145, 32 186; of 2048 rows K=32 222, 48 249; of 2050 rows
+//    K=48 253, one thread per line 1829; of 4096 rows (K = 48, 4 columns)
+//    1081, one thread per line 3820.
+template <typename T>
+int z_default(int n3m, int nwg16) {
+    if (n3m > 2048) return n3m <= 3072 ? kZLong8 : kZLong4;
+    if (n3m > 1024) return n3m <= 1536 ? 14 : 4;
+    if (nwg16 < 4 * num_cus()) return n3m <= 400 ? 5 : (n3m <= 512 ? 2 : (n3m <= 768 ? 13 : 4));
+    if (n3m <= 24) return 11;
+    if (sizeof(T) == 4 && n3m <= 256) return n3m <= 128 ? 16 : 15;
+    if (n3m <= 64) return 1;
+    if (n3m <= 128) return 11;
+    if (n3m <= 320) return 7;
+    if (n3m <= 384) return 12;
+    if (n3m <= 448) return 17;
+    if (n3m <= 512) return 3;
+    return n3m <= 768 ? 12 : 3;
+}
+}  // namespace
+
 template <typename T>
 int launch_z(ppf_plan *p, T *W, const double *dx3, const double *dmx3, hipStream_t s) {
-    // k_zpart and k_zpipe read the z row table that pass 1 of this solve filled
+    // k_zpart reads the z row table that pass 1 of this solve filled
     ZArgs z;
     z.Lx = p->Lx;
     z.Lxs = p->Lxs;
@@ -29,16 +70,15 @@ int launch_z(ppf_plan *p, T *W, const double *dx3, const double *dmx3, hipStream
     z.gate = p->gate;
     const int n3m = p->d.n3m;
     // partitioned register-resident Thomas, shape (K rows per thread, S
-    // columns per workgroup); launched only when S*P <= NTMAX and the LDS
-    // footprint stays within 64 KiB, else the one-thread-per-line kernel
+    // columns per workgroup); launched only when S*P <= NTMAX, the LDS
+    // footprint stays within `lds` and n3m within `most`
     bool done = false;
-    auto part = [&](auto kk, auto ss, auto nt, auto wpe) {
+    auto part = [&](auto kk, auto ss, auto nt, auto wpe, int most = 4096, size_t lds = 65536) {
         constexpr int K = decltype(kk)::value, S = decltype(ss)::value;
         constexpr int NTMAX = decltype(nt)::value, WPE = decltype(wpe)::value;
         const int P = (n3m + K - 1) / K;
-        constexpr int KS = (K + S - 1) / S;  // z table rows per thread
-        const size_t shm = sizeof(double) * (2 * (size_t)KS * S * P + 7 * (size_t)P * S);
-        if (P < 1 || S * P > NTMAX || shm > 65536) return;
+        const size_t shm = zp_lds_bytes<K, S>(P);
+        if (P < 1 || S * P > NTMAX || shm > lds || n3m > most) return;
         const int tiles = (p->Lx + S - 1) / S;
         const int ntiles = tiles * p->znjr;
         // FP64 arithmetic for FP32 storage too: FP32 arithmetic measured no
@@ -47,50 +87,36 @@ int launch_z(ppf_plan *p, T *W, const double *dx3, const double *dmx3, hipStream
                            p->zcoef, p->zcoef + n3m, p->mean, P);
         done = true;
     };
-    // pipelined variant: persistent, prefetching, wavefront cyclic reduction
-    auto pipe = [&](auto kk, auto ss, auto wpe) {
-        constexpr int K = decltype(kk)::value, S = decltype(ss)::value, WPE = decltype(wpe)::value;
-        const int P = (n3m + K - 1) / K;
-        const size_t shm = sizeof(double) * (2 * (size_t)P * K + 3 * (size_t)S * 65 + (size_t)P * S);
-        if (P < 1 || P > 32 || K < 2 || shm > 65536) return;
-        const double *zam = p->zcoef, *zap = p->zcoef + n3m;
-        const int ntiles = ((p->Lx + S - 1) / S) * p->znjr;
-        const unsigned g = persistent_grid(k_zpipe<T, K, S, WPE>, S * P, ntiles, shm);
-        hipLaunchKernelGGL((k_zpipe<T, K, S, WPE>), dim3(g), dim3(S * P), shm, s, W, z, zam, zap, p->mean, P);
-        done = true;
-    };
     using std::integral_constant;
-    int v = p->zvariant;
-    // measured on MI355X at 512^3: (K=32, S=16) 0.54 ms, pipelined K=16 0.81 ms
-    if (v == 0) v = (n3m <= 1024) ? 3 : 4;
-    // the pipelined form writes wall ghost planes only
-    if (z.zper && ((v >= 7 && v <= 11) || v == 17)) v = (n3m <= 1024) ? 3 : 4;
+#define PPF_Z(K, S, NT, WPE) integral_constant<int, K>{}, integral_constant<int, S>{}, integral_constant<int, NT>{}, integral_constant<int, WPE>{}
+    int v = p->zvariant ? p->zvariant : z_default<T>(n3m, (p->Lx + 15) / 16 * p->znjr);
+    // with periodic z a pin of the shapes below whose extent is limited means
+    // the shape without that limit
+    if (z.zper && ((v >= 7 && v <= 11) || v == 17) && p->zvariant) v = n3m <= 1024 ? 3 : 4;
     switch (v) {
-        case 7: pipe(integral_constant<int, 16>{}, integral_constant<int, 16>{}, integral_constant<int, 2>{}); break;
-        case 8: pipe(integral_constant<int, 16>{}, integral_constant<int, 8>{}, integral_constant<int, 2>{}); break;
-        case 9: pipe(integral_constant<int, 32>{}, integral_constant<int, 8>{}, integral_constant<int, 2>{}); break;
-        case 10: pipe(integral_constant<int, 32>{}, integral_constant<int, 16>{}, integral_constant<int, 2>{}); break;
-        case 11: pipe(integral_constant<int, 8>{}, integral_constant<int, 16>{}, integral_constant<int, 4>{}); break;
-        case 17: pipe(integral_constant<int, 24>{}, integral_constant<int, 16>{}, integral_constant<int, 2>{}); break;
-        default: break;
-    }
-    switch (v) {
-        case 1: part(integral_constant<int, 16>{}, integral_constant<int, 16>{}, integral_constant<int, 512>{}, integral_constant<int, 3>{}); break;
-        case 2: part(integral_constant<int, 16>{}, integral_constant<int, 8>{}, integral_constant<int, 512>{}, integral_constant<int, 3>{}); break;
-        case 3: part(integral_constant<int, 32>{}, integral_constant<int, 16>{}, integral_constant<int, 512>{}, integral_constant<int, 2>{}); break;
-        case 4: part(integral_constant<int, 32>{}, integral_constant<int, 8>{}, integral_constant<int, 512>{}, integral_constant<int, 2>{}); break;
-        case 5: part(integral_constant<int, 8>{}, integral_constant<int, 8>{}, integral_constant<int, 512>{}, integral_constant<int, 4>{}); break;
-        case 12: part(integral_constant<int, 24>{}, integral_constant<int, 16>{}, integral_constant<int, 512>{}, integral_constant<int, 2>{}); break;
-        case 13: part(integral_constant<int, 24>{}, integral_constant<int, 8>{}, integral_constant<int, 512>{}, integral_constant<int, 2>{}); break;
-        case 14: part(integral_constant<int, 48>{}, integral_constant<int, 8>{}, integral_constant<int, 512>{}, integral_constant<int, 1>{}); break;
+        case 1: part(PPF_Z(16, 16, 512, 4)); break;
+        case 2: part(PPF_Z(16, 8, 512, 4)); break;
+        case 3: case 10: part(PPF_Z(32, 16, 512, 3)); break;
+        case 4: case 9: part(PPF_Z(32, 8, 512, 3), v == 9 ? 1024 : 4096); break;
+        case 5: part(PPF_Z(8, 8, 512, 4)); break;
+        case 7: part(PPF_Z(20, 16, 512, 4), 512); break;
+        case 8: part(PPF_Z(12, 16, 704, 4), 512); break;
+        case 11: part(PPF_Z(8, 16, 512, 4)); break;
+        case 12: part(PPF_Z(24, 16, 512, 4)); break;
+        case 13: part(PPF_Z(24, 8, 512, 3)); break;
+        case 14: part(PPF_Z(48, 8, 512, 2)); break;
         // 32 columns: 128-byte row segments for FP32 workspaces
-        case 15: part(integral_constant<int, 32>{}, integral_constant<int, 32>{}, integral_constant<int, 512>{}, integral_constant<int, 2>{}); break;
-        case 16: part(integral_constant<int, 16>{}, integral_constant<int, 32>{}, integral_constant<int, 512>{}, integral_constant<int, 3>{}); break;
+        case 15: part(PPF_Z(32, 32, 512, 3)); break;
+        case 16: part(PPF_Z(16, 32, 512, 4)); break;
+        case 17: part(PPF_Z(28, 16, 512, 3), 768); break;
+        // lines over 2048 rows (not selectable)
+        case kZLong8: part(PPF_Z(48, 8, 512, 2), 3072, 160 * 1024); break;
+        case kZLong4: part(PPF_Z(48, 4, 512, 2), 4096, 160 * 1024); break;
         default: break;
     }
-    // a pinned shape that does not fit the extent is reported, never replaced:
-    // only the default (v chosen above) and shape 6 fall to one thread per line
-    if (!done && p->zvariant != 0 && p->zvariant != 6) return PPF_ERR_UNSUPPORTED;
+#undef PPF_Z
+    // a pinned shape that does not fit the extent is reported, never replaced
+    if (!done && v != 6) return PPF_ERR_UNSUPPORTED;
     if (!done) {
         const long ncol = (long)p->Lx * p->znjr;
         // the one-thread-per-line kernel keeps its forward multipliers in cs

@@ -1,0 +1,54 @@
+"""The z-pass shape of a plan that was not tuned, at the line lengths where the
+rule changes shape, on a small grid (few workgroups: 8-column shapes) and on one
+with four 16-column workgroups per CU, against the FP64 oracle.
+
+FP64 plans are held to 1e-12 up to 512 rows and to 1e-11 above: the pinned
+(0,0) line is ill conditioned, and the oracle's own FP64 Thomas on it is off an
+80-bit solve of these inputs by up to 0.5e-12 of the whole solution at 514 rows
+and 1.06e-12 at 770 (0.16e-12 at 512), so that two correct FP64 algorithms may
+differ by a few times that.  FP32_IR plans
+run one FP32 solve without corrections: storage rounding is 6e-8 a pass over
+five passes, relative to the largest values of a field whose smallest modes
+dominate, so 5e-6 bounds it and a wrong row or mask (order one) does not pass.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from pascal_poisson_fft_amd import api
+from pascal_poisson_fft_amd.grid import make_axis
+
+pytestmark = pytest.mark.gpu
+
+SMALL = [8, 24, 26, 400, 402, 512, 514, 768, 770, 1024, 1026, 1536, 1538, 2048, 2050, 3072, 3074, 4096]
+LARGE = [4, 24, 26, 64, 66, 128, 130, 256, 258, 320, 322, 384, 386, 448, 450, 512, 514, 768, 770, 1022]
+
+
+def _solve(n1, n2, n3, pbc, precision):
+    L = (2.0, 3.0, 1.5)
+    ax, ay = make_axis(n1, L[0], pbc[0]), make_axis(n2, L[1], pbc[1])
+    az = make_axis(n3, L[2], False, uniform=False, gamma=1.6)
+    f = np.random.default_rng(n1 + n3).standard_normal((n3, n2, n1))
+    f -= float(np.einsum("kji,k->", f, az.dx[1:n3 + 1])) / (az.dx[1:n3 + 1].sum() * n1 * n2)
+    ref = O.solve(f, L, (pbc[0], pbc[1], False), ax.dmx, ay.dmx, az.dmx, az.dx)
+    plan = api.FFTPoisson(n1, n2, n3, L, (pbc[0], pbc[1], False), precision=precision)
+    dev = api.Problem3D(f, ax, ay, az)
+    try:
+        args = (dev.rhs, dev.p, dev.dmx1, dev.dmx2, dev.dmx3, dev.dx3)
+        plan.solve_sweeps(*args, 0)
+        api.sync()
+        got = dev.p.download()
+    finally:
+        dev.free()
+        plan.clean()
+    return float(np.linalg.norm(got - ref) / np.linalg.norm(ref))
+
+
+@pytest.mark.parametrize("precision", [api.PPF_PREC_FP64, api.PPF_PREC_FP32_IR], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("n1,n2,n3", [(20, 12, n) for n in SMALL] + [(160, 120, n) for n in LARGE])
+def test_default_z_shape_matches_oracle(n1, n2, n3, precision):
+    # 20 columns, and the 162 of periodic x, leave a ragged last column tile
+    pbc = (n3 % 4 == 2, n3 % 8 >= 4)
+    err = _solve(n1, n2, n3, pbc, precision)
+    bar = (1e-12 if n3 <= 512 else 1e-11) if precision == api.PPF_PREC_FP64 else 5e-6
+    assert err <= bar, err
