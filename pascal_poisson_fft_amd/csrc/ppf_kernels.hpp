@@ -146,11 +146,38 @@ constexpr int x_line_pad(int s) {
     return ((128 - base + 256) % 256) / (int)sizeof(T);
 }
 
+// complex values a thread holds in the widest stage of an M-point line with
+// tpl threads
+constexpr int stage_values(int m, int tpl) {
+    int most = 0;
+    for (int rem = m; rem > 1;) {
+        const int r = pick_radix(rem), v = (m / r + tpl - 1) / tpl * r;
+        most = v > most ? v : most;
+        rem /= r;
+    }
+    return most;
+}
+// threads of an x line: the smallest power of two that leaves a thread one
+// widest butterfly's worth of values, at most 8
+constexpr int x_line_threads(int m) {
+    int p = 1;
+    while (p < m / max_radix(m) || stage_values(m, p) > 8) p *= 2;
+    return p;
+}
 template <typename T, int N, bool PER, int XV = 0>
 struct XGeom {
     using G = LineGeom<N, PER>;
     static constexpr bool LITE = XV == 2;
-    static constexpr int TPL = (G::TPL >> (XV == 1 ? 1 : 0)) > 0 ? (G::TPL >> (XV == 1 ? 1 : 0)) : 1;
+    // threads per line: a power of two, so that LPB lines times PT lanes divide
+    // the workgroup and a thread keeps one line of the tile on the W side
+    // (ONE_ROW).  With M / max_radix threads (20 for 320 points) every pair of
+    // the W side took its own line and address arithmetic, which then bounded
+    // the pass: 16.8M cells, N-N, forward / inverse us: 320 points 109 / 135 ->
+    // 56 / 68, 192 points 106 / 137 -> 57 / 67, 112 points 130 / 150 -> 54 /
+    // 63.  The bound of 8 values matters to 240 and 960 points: without
+    // it 120 / 87 and 165 / 125, with it 60 / 71 and 63 / 74.
+    static constexpr int TPL2 = x_line_threads(G::M);
+    static constexpr int TPL = (TPL2 >> (XV == 1 ? 1 : 0)) > 0 ? (TPL2 >> (XV == 1 ? 1 : 0)) : 1;
     static constexpr int LPB = (256 / TPL) > 0 ? (256 / TPL) : 1;
     static constexpr int NT = LPB * TPL;
     // the bank pad where a thread keeps one line per tile (the longer lines:
