@@ -22,89 +22,162 @@ struct ppf_tdma_plan {
 
 namespace {
 
-__global__ void __launch_bounds__(256)
-k_tdma_many(const double *__restrict__ a, const double *__restrict__ b, double *__restrict__ c, double *__restrict__ d,
-            long nsys, int nrow) {
+// One thread solves one system, row after row, so what bounds these kernels is
+// the latency of a row's loads unless they are issued ahead: rows come in
+// chunks of U, the next chunk's loads in flight while the current one is
+// eliminated, and a chunk's stores are younger than the loads that follow it
+// in the chain, so nothing waits for them.  One-wave workgroups spread a few
+// thousand systems over as many CUs as there are waves.  256^3 (many systems):
+// 291 -> 200 us, 6.0 TB/s of the 72 bytes a row moves; cyclic 100 x 60 systems
+// of 90 rows: 69 -> 34 us and 256 systems of 512 rows 242 -> 107 us, where a
+// row's chain of a correctly rounded division and the products that use it
+// (about 0.2 us) is what is left.  16 rows a forward chunk were no faster (205,
+// 34, 101 us), 8 rows a backward chunk neither (200, 36, 113).
+constexpr int kTdmaThreads = 64;
+constexpr int kTdmaFwd = 8;    // rows a chunk of the elimination: 4 arrays x 8 rows x 2 chunks = 128 registers
+constexpr int kTdmaBack = 16;  // of the substitutions, whose rows take less time than their loads' latency
+
+// U rows of the N arrays src, from row k0 in steps of DIR, clamped to the ends
+template <int N, int U, int DIR>
+struct TdmaRows {
+    double v[N][U];
+    __device__ __forceinline__ void load(const double *const (&src)[N], size_t ns, long s, int k0, int nrow) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = DIR > 0 ? (k0 + u < nrow ? k0 + u : nrow - 1) : (k0 - u > 0 ? k0 - u : 0);
+#pragma unroll
+            for (int n = 0; n < N; ++n) v[n][u] = src[n][(size_t)k * ns + s];
+        }
+    }
+};
+
+__global__ void __launch_bounds__(kTdmaThreads)
+k_tdma_many(const double *__restrict__ a, const double *__restrict__ b, double *c, double *d, long nsys, int nrow) {
 #pragma clang fp contract(off)
     const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= nsys) return;
-    double dp = d[s] / b[s];
-    double cp = c[s] / b[s];
-    d[s] = dp;
-    c[s] = cp;
-    for (int k = 1; k < nrow; ++k) {
-        const size_t q = (size_t)k * (size_t)nsys + (size_t)s;
-        const double ak = a[q];
-        const double r = 1.0 / (b[q] - ak * cp);
-        dp = r * (d[q] - ak * dp);
-        cp = r * c[q];
-        d[q] = dp;
-        c[q] = cp;
+    constexpr int U = kTdmaFwd, V = kTdmaBack;
+    const size_t ns = (size_t)nsys;
+    double dp, cp;
+    {
+        const double *const src[4] = {a, b, c, d};
+        TdmaRows<4, U, 1> cur, nxt;
+        cur.load(src, ns, s, 1, nrow);
+        dp = d[s] / b[s];
+        cp = c[s] / b[s];
+        d[s] = dp;
+        c[s] = cp;
+        for (int k0 = 1; k0 < nrow; k0 += U) {
+            if (k0 + U < nrow) nxt.load(src, ns, s, k0 + U, nrow);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (k0 + u < nrow) {
+                    const size_t q = (size_t)(k0 + u) * ns + (size_t)s;
+                    const double ak = cur.v[0][u];
+                    const double r = 1.0 / (cur.v[1][u] - ak * cp);
+                    dp = r * (cur.v[3][u] - ak * dp);
+                    cp = r * cur.v[2][u];
+                    d[q] = dp;
+                    c[q] = cp;
+                }
+            }
+            cur = nxt;
+        }
     }
-    for (int k = nrow - 2; k >= 0; --k) {
-        const size_t q = (size_t)k * (size_t)nsys + (size_t)s;
-        dp = d[q] - c[q] * dp;
-        d[q] = dp;
+    const double *const src[2] = {c, d};
+    TdmaRows<2, V, -1> cur, nxt;
+    cur.load(src, ns, s, nrow - 2, nrow);
+    for (int k0 = nrow - 2; k0 >= 0; k0 -= V) {
+        if (k0 - V >= 0) nxt.load(src, ns, s, k0 - V, nrow);
+#pragma unroll
+        for (int u = 0; u < V; ++u) {
+            if (k0 - u >= 0) {
+                dp = cur.v[1][u] - cur.v[0][u] * dp;
+                d[(size_t)(k0 - u) * ns + (size_t)s] = dp;
+            }
+        }
+        cur = nxt;
     }
 }
 
 // Cyclic Thomas, op order of tdma_cycl_many_cuda (tdmas_cuda.f90:114-217):
 // rows 1..n-1 are reduced for d' and the correction vector e (e_1 = -a_1,
-// e_{n-1} = -c_{n-1}), x_0 follows from row 0, then x_k = d'_k + x_0 e_k.
-// The reference keeps d'_1, e'_1 for row 0 in shared-memory registers after
-// the backward loop; they are re-read here (same values, and defined for
-// n = 2, where the reference's backward loop never sets them).
-__global__ void __launch_bounds__(256)
-k_tdma_cycl_many(const double *__restrict__ a, const double *__restrict__ b, double *__restrict__ c,
-                 double *__restrict__ d, double *__restrict__ e, long nsys, int nrow) {
+// e_{n-1} = -c_{n-1}, zero between: constants here, not stored and read back),
+// x_0 follows from row 0, then x_k = d'_k + x_0 e_k.  x_0 uses rows 1 and n-1 of d and e after the backward loop, which for
+// n = 2 (one row) are the forward values.
+__global__ void __launch_bounds__(kTdmaThreads)
+k_tdma_cycl_many(const double *__restrict__ a, const double *__restrict__ b, double *c, double *d, double *e, long nsys,
+                 int nrow) {
 #pragma clang fp contract(off)
     const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= nsys) return;
+    constexpr int U = kTdmaFwd, V = kTdmaBack;
     const size_t ns = (size_t)nsys;
-    for (int k = 0; k < nrow; ++k) e[(size_t)k * ns + s] = 0.0;
-    e[ns + s] = -a[ns + s];
-    e[(size_t)(nrow - 1) * ns + s] = -c[(size_t)(nrow - 1) * ns + s];
-    double d1 = d[ns + s], b1 = b[ns + s], c1 = c[ns + s], e1 = e[ns + s];
-    d1 = d1 / b1;
-    c1 = c1 / b1;
-    e1 = e1 / b1;
-    d[ns + s] = d1;
-    c[ns + s] = c1;
-    e[ns + s] = e1;
-    for (int k = 2; k < nrow; ++k) {
-        const size_t q = (size_t)k * ns + s;
-        const double c0 = c1, d0 = d1, e0 = e1;
-        const double ak = a[q];
-        b1 = b[q];
-        c1 = c[q];
-        d1 = d[q];
-        e1 = e[q];
-        const double r = 1.0 / (b1 - ak * c0);
-        d1 = r * (d1 - ak * d0);
-        e1 = r * (e1 - ak * e0);
-        c1 = r * c1;
-        e[q] = e1;
-        d[q] = d1;
-        c[q] = c1;
+    const int last = nrow - 1;
+    const double a0 = a[s], b0 = b[s], c0 = c[s], d0 = d[s];
+    double d1 = d[ns + s], b1 = b[ns + s], c1 = c[ns + s], e1 = last == 1 ? -c1 : -a[ns + s];
+    {
+        const double *const src[4] = {a, b, c, d};
+        TdmaRows<4, U, 1> cur, nxt;
+        cur.load(src, ns, s, 2, nrow);
+        d1 = d1 / b1;
+        c1 = c1 / b1;
+        e1 = e1 / b1;
+        d[ns + s] = d1;
+        c[ns + s] = c1;
+        e[ns + s] = e1;
+        for (int k0 = 2; k0 < nrow; k0 += U) {
+            if (k0 + U < nrow) nxt.load(src, ns, s, k0 + U, nrow);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int k = k0 + u;
+                if (k < nrow) {
+                    const size_t q = (size_t)k * ns + (size_t)s;
+                    const double ak = cur.v[0][u];
+                    const double ek = k == last ? -cur.v[2][u] : 0.0;
+                    const double r = 1.0 / (cur.v[1][u] - ak * c1);
+                    d1 = r * (cur.v[3][u] - ak * d1);
+                    e1 = r * (ek - ak * e1);
+                    c1 = r * cur.v[2][u];
+                    e[q] = e1;
+                    d[q] = d1;
+                    c[q] = c1;
+                }
+            }
+            cur = nxt;
+        }
     }
-    for (int k = nrow - 2; k >= 1; --k) {
-        const size_t q = (size_t)k * ns + s;
-        double c0 = c[q], d0 = d[q], e0 = e[q];
-        d0 = d0 - c0 * d1;
-        e0 = e0 - c0 * e1;
-        d1 = d0;
-        e1 = e0;
-        d[q] = d0;
-        e[q] = e0;
+    const double dn = d1, en = e1;  // row n-1
+    {
+        const double *const src[3] = {c, d, e};
+        TdmaRows<3, V, -1> cur, nxt;
+        cur.load(src, ns, s, nrow - 2, nrow);
+        for (int k0 = nrow - 2; k0 >= 1; k0 -= V) {
+            if (k0 - V >= 1) nxt.load(src, ns, s, k0 - V, nrow);
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                if (k0 - u >= 1) {
+                    const size_t q = (size_t)(k0 - u) * ns + (size_t)s;
+                    d1 = cur.v[1][u] - cur.v[0][u] * d1;
+                    e1 = cur.v[2][u] - cur.v[0][u] * e1;
+                    d[q] = d1;
+                    e[q] = e1;
+                }
+            }
+            cur = nxt;
+        }
     }
-    const size_t qn = (size_t)(nrow - 1) * ns + s;
-    const double a0 = a[s], b0 = b[s], c0 = c[s];
-    double x0 = d[s];
-    x0 = (x0 - a0 * d[qn] - c0 * d[ns + s]) / (b0 + a0 * e[qn] + c0 * e[ns + s]);
+    const double x0 = (d0 - a0 * dn - c0 * d1) / (b0 + a0 * en + c0 * e1);
     d[s] = x0;
-    for (int k = 1; k < nrow; ++k) {
-        const size_t q = (size_t)k * ns + s;
-        d[q] = d[q] + x0 * e[q];
+    const double *const src[2] = {d, e};
+    TdmaRows<2, V, 1> cur, nxt;
+    cur.load(src, ns, s, 1, nrow);
+    for (int k0 = 1; k0 < nrow; k0 += V) {
+        if (k0 + V < nrow) nxt.load(src, ns, s, k0 + V, nrow);
+#pragma unroll
+        for (int u = 0; u < V; ++u)
+            if (k0 + u < nrow) d[(size_t)(k0 + u) * ns + (size_t)s] = cur.v[0][u] + x0 * cur.v[1][u];
+        cur = nxt;
     }
 }
 
@@ -131,7 +204,7 @@ int ppf_tdma_plan_many_create(int nx_sys, int ny_sys, int nz_row, ppf_tdma_plan 
 int ppf_tdma_many_solve(ppf_tdma_plan *p, const double *a, const double *b, double *c, double *d, void *stream) {
     if (!p || !a || !b || !c || !d) return PPF_ERR_INVALID_ARG;
     const long nsys = (long)p->nx * p->ny;
-    const int nt = 256;
+    const int nt = kTdmaThreads;
     hipLaunchKernelGGL(k_tdma_many, dim3((unsigned)((nsys + nt - 1) / nt)), dim3(nt), 0,
                        static_cast<hipStream_t>(stream), a, b, c, d, nsys, p->nz);
     return hipGetLastError() == hipSuccess ? PPF_OK : PPF_ERR_HIP;
@@ -142,7 +215,7 @@ int ppf_tdma_many_solve_cycle(ppf_tdma_plan *p, const double *a, const double *b
     if (!p || !a || !b || !c || !d) return PPF_ERR_INVALID_ARG;
     if (p->nz < 2) return PPF_ERR_SIZE;
     const long nsys = (long)p->nx * p->ny;
-    const int nt = 256;
+    const int nt = kTdmaThreads;
     hipLaunchKernelGGL(k_tdma_cycl_many, dim3((unsigned)((nsys + nt - 1) / nt)), dim3(nt), 0,
                        static_cast<hipStream_t>(stream), a, b, c, d, p->e, nsys, p->nz);
     return hipGetLastError() == hipSuccess ? PPF_OK : PPF_ERR_HIP;
