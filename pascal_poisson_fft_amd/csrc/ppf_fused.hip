@@ -271,11 +271,9 @@ int fused_residual(ppf_fused *f, int i, hipStream_t s, double *rel) {
     xr.ih2 = 1.0 / (h2 * h2);
     xr.pbc1 = d.pbc1 != 0;
     xr.pbc2 = d.pbc2 != 0;
-    const int ty = residual_rows(d.n1m, d.n2m, d.n3m, 4L * num_cus());
-    const long ntiles = residual_tiles(d.n1m, d.n2m, d.n3m, ty);
-    const int g = (int)std::min<long>(std::min<long>(kResPartials, 8L * num_cus()), ntiles);
-    launch_k_residual(ty, g, s, q.in, xr, d.n1m, d.n2m, d.n3m, nullptr);
-    hipLaunchKernelGGL(k_reduce3, dim3(1), dim3(256), 0, s, f->partial, g, f->red, nullptr);
+    const ResShape rs = residual_shape(d.n1m, d.n2m, d.n3m, num_cus(), kResPartials);
+    launch_k_residual(rs, s, q.in, xr, d.n1m, d.n2m, d.n3m, nullptr);
+    hipLaunchKernelGGL(k_reduce3, dim3(1), dim3(256), 0, s, f->partial, (int)rs.grid, f->red, nullptr);
     PPF_HIP(hipGetLastError());
     double hr[3];
     PPF_HIP(hipStreamSynchronize(s));

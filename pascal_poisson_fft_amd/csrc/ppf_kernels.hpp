@@ -21,6 +21,8 @@
 //   pass 5  x-inverse   W rows    -> P            + x ghosts, mean removal
 #pragma once
 
+#include <algorithm>
+
 #include "ppf_lines.hpp"
 
 namespace ppf {
@@ -1409,19 +1411,21 @@ k_zpart(T *__restrict__ W, ZArgs z, const double *__restrict__ zam, const double
 // of XRes), with per-workgroup sums of r^2, f^2 and p (deterministic
 // two-level reduction with k_reduce3); with xr.rout set, r is also stored in
 // FP32 in the W row pass 1 transforms next (the refinement sweep's input).
-// A tile is 256 consecutive x cells of TY consecutive rows j (TY divides n2m)
-// over KZ consecutive planes.  Each thread walks its TY columns up the planes
-// keeping p(k-1), p(k), p(k+1) of all TY rows in registers:
+// A tile is one wave's: 64 consecutive x cells of TY consecutive rows j (TY
+// divides n2m) over kz consecutive planes.  A lane walks its TY cells up the
+// planes keeping p(k-1), p(k), p(k+1) in registers:
 //  * y neighbours inside the block come from those registers; only the two
 //    halo rows (j0-1 and j0+TY, or the wall row itself, or the periodic
 //    wrap) are loaded;
 //  * x neighbours come from the adjacent lanes of the wavefront (DPP wave
-//    shifts); only a wave's edge lanes and the domain's edge cells load them;
+//    shifts); only a wave's two edge lanes load theirs, one masked load a row;
 //  * the tiles of one XCD (workgroup b runs on XCD b mod 8) are consecutive,
 //    so a halo row is usually in that XCD's L2 already.
-// P is fetched about 1.1 times at 512^3 (one row per thread, with x and y
-// neighbours loaded, fetched it about 2.7 times: 35 against 16 B per cell,
-// 0.70 against 0.49 ms).  Workgroups stride over the tiles.
+// The loads of plane k+1, edge cells included, are issued before the stores of
+// plane k: one counter covers loads and stores, in order, so loads issued
+// after the stores made every plane wait for the stores to reach memory
+// (512^3: 741 -> 540 us with the store, 481 -> 410 without, 5.2-5.8 TB/s of
+// the bytes moved; 2 to 4 waves per SIMD make no difference there).  Workgroups stride over the tiles.
 // ---------------------------------------------------------------------------
 // value of lane l-1 (l+1) of the wavefront: DPP wave_shr:1 (wave_shl:1) per dword
 __device__ __forceinline__ double dpp_lane_minus1(double v) {
@@ -1437,89 +1441,118 @@ __device__ __forceinline__ double dpp_lane_plus1(double v) {
     return __builtin_bit_cast(double, r);
 }
 
-template <int KZ, int TY, bool STORE>
-__global__ void __launch_bounds__(256)
-k_residual(const double *__restrict__ f, XRes xr, int n1m, int n2m, int n3m, const int *__restrict__ gate) {
+template <int TY, bool STORE>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TY == 8 ? 4 : 1)))
+k_residual(const double *__restrict__ f, XRes xr, int n1m, int n2m, int n3m, int kz, const int *__restrict__ gate) {
     if (gated_off(gate)) return;
     __shared__ double red[256];
-    const int nxc = (n1m + 255) / 256, nyb = n2m / TY, nkb = (n3m + KZ - 1) / KZ;
+    const int nxc = (n1m + 63) / 64, nyb = n2m / TY, nkb = (n3m + kz - 1) / kz;
     const long ntiles = (long)nxc * nyb * nkb;
     const long L1 = (long)n1m + 2, L2 = (long)n2m + 2, pl = L1 * L2;
     const double *__restrict__ P = xr.P;
     double sr = 0.0, sf = 0.0, sx = 0.0;
+    const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     // XCD-grouped tile order (a permutation of the workgroups when 8 | grid)
     const long vb = (gridDim.x % 8 == 0) ? (long)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
-    for (long tile = vb; tile < ntiles; tile += gridDim.x) {
+    for (long tile = vb * 4 + wave; tile < ntiles; tile += (long)gridDim.x * 4) {
         const int xc = (int)(tile % nxc);
         const long rest = tile / nxc;
         const int jb = (int)(rest % nyb), kb = (int)(rest / nyb);
-        const int i = xc * 256 + (int)threadIdx.x;
-        if (i >= n1m) continue;
-        // x neighbour offsets: zero-flux walls reuse the centre, periodic x wraps
-        long dxm = -1, dxp = 1;
-        if (xr.pbc1) {
-            if (i == 0) dxm = n1m - 1;
-            if (i == n1m - 1) dxp = -(long)(n1m - 1);
-        } else {
-            if (i == 0) dxm = 0;
-            if (i == n1m - 1) dxp = 0;
-        }
-        const int lane = (int)threadIdx.x & 63;
-        const bool xedge_m = lane == 0 || i == 0, xedge_p = lane == 63 || i == n1m - 1;
+        // lanes past the last cell load it again and are masked out
+        const bool act = xc * 64 + lane < n1m;
+        const int i = act ? xc * 64 + lane : n1m - 1;
+        // edge lanes (n1m is even, so they are distinct): the outer x neighbour;
+        // zero-flux walls reuse the centre, periodic x wraps
+        const bool edge_m = lane == 0, edge_p = act && (lane == 63 || i == n1m - 1);
+        int ie = i;
+        if (edge_m) ie = i > 0 ? i - 1 : (xr.pbc1 ? n1m - 1 : 0);
+        if (edge_p) ie = i < n1m - 1 ? i + 1 : (xr.pbc1 ? 0 : n1m - 1);
         // halo rows of the block: the row below j0 and the row above j0+TY-1
         // (at a wall the edge row itself, for periodic y the wrapped row)
         const int j0 = jb * TY;
         const int jlo = j0 > 0 ? j0 - 1 : (xr.pbc2 ? n2m - 1 : 0);
         const int jhi = j0 + TY < n2m ? j0 + TY : (xr.pbc2 ? 0 : n2m - 1);
         const long dlo = (long)(jlo - j0) * L1, dhi = (long)(jhi - j0) * L1;
-        const int k0 = kb * KZ;
-        const long pc0 = ((long)(k0 + 1) * L2 + (j0 + 1)) * L1 + (i + 1);
-        double zm[TY], c[TY];  // planes k-1 and k of the TY rows
+        const int k0 = kb * kz, k1 = k0 + kz < n3m ? k0 + kz : n3m;
+        // row starts are uniform over the wave (scalar registers); a lane adds
+        // its own 32-bit position in the row
+        const double *pp = P + ((long)(k0 + 1) * L2 + (j0 + 1)) * L1;  // row j0 of plane k
+        const double *fp = f + ((long)k0 * n2m + j0) * n1m;
+        const unsigned u = (unsigned)i + 1, ue = (unsigned)ie + 1;
+        double zm[TY], c[TY], zp[TY], fv[TY], xe[TY], hlo, hhi;  // planes k-1, k, k+1, f, the outer x neighbours, halos
+        auto load = [&]() {  // what plane k needs beside zm and c
+            // row starts are stepped here, not kept over the loop: the scalar
+            // registers do not hold them all
+            long l1 = L1, m1 = n1m;
+            asm volatile("" : "+s"(l1), "+s"(m1));
+            const double *q = pp + pl;
+#pragma unroll
+            for (int t = 0; t < TY; ++t, q += l1) zp[t] = q[u];
+            hlo = (pp + dlo)[u];
+            hhi = (pp + dhi)[u];
+            if (edge_m || edge_p) {
+                q = pp;
+#pragma unroll
+                for (int t = 0; t < TY; ++t, q += l1) xe[t] = q[ue];
+            }
+            q = fp;
+#pragma unroll
+            for (int t = 0; t < TY; ++t, q += m1) fv[t] = ld_stream(q + (unsigned)i);
+        };
 #pragma unroll
         for (int t = 0; t < TY; ++t) {
-            zm[t] = P[pc0 + t * L1 - pl];  // ghost plane below the first (finite, weight 0 at the wall)
-            c[t] = P[pc0 + t * L1];
+            zm[t] = (pp + t * L1 - pl)[u];  // ghost plane below the first (finite, weight 0 at the wall)
+            c[t] = (pp + t * L1)[u];
+            xe[t] = 0.0;
         }
-        // planes past n3m load the last plane again (clamped addresses, no
-        // branch); their terms are masked out of the sums
-#pragma unroll 2
-        for (int kk = 0; kk < KZ; ++kk) {
-            const int k0k = k0 + kk;
-            const bool in = k0k < n3m;
-            const int k = in ? k0k : n3m - 1;
-            const long pc = pc0 + (long)(k - k0) * pl;
-            double zp[TY];
-#pragma unroll
-            for (int t = 0; t < TY; ++t) zp[t] = P[pc + t * L1 + pl];
-            const double hlo = P[pc + dlo], hhi = P[pc + dhi];
+        load();
+        // STORE: r of row j0+t goes to W32 plane k+1, row j0+t+1 (rows of a
+        // column tile are one tile width apart)
+        float *rrow = nullptr;
+        unsigned ru = 0;
+        if constexpr (STORE) {
+            rrow = xr.rout + (size_t)(k0 + 1) * (size_t)xr.Ly * (size_t)xr.Lxs + (size_t)(j0 + 1) * w_tile<float>();
+            ru = (unsigned)w_col<float>(i, xr.Ly);
+        }
+        for (int k = k0; k < k1; ++k) {
             const double am = xr.zam[k], ap = xr.zap[k];
-            // STORE: r of row j0+t goes to W32 plane k+1, row j0+t+1 (rows of a
-            // column tile are one tile width apart)
-            float *rrow = nullptr;
-            if constexpr (STORE)
-                rrow = xr.rout + (size_t)(k + 1) * (size_t)xr.Ly * (size_t)xr.Lxs + w_at<float>(j0 + 1, i, xr.Ly);
+            float rs[TY];
 #pragma unroll
             for (int t = 0; t < TY; ++t) {
-                const long q = pc + t * L1;
                 double xm = dpp_lane_minus1(c[t]), xp = dpp_lane_plus1(c[t]);
-                if (xedge_m) xm = P[q + dxm];
-                if (xedge_p) xp = P[q + dxp];
+                xm = edge_m ? xe[t] : xm;
+                xp = edge_p ? xe[t] : xp;
                 const double ym = t > 0 ? c[t - 1] : hlo, yp = t < TY - 1 ? c[t + 1] : hhi;
-                const double fv = ld_stream(&f[((size_t)k * n2m + (j0 + t)) * n1m + i]);
                 const double lp = (xp - 2.0 * c[t] + xm) * xr.ih1 + (yp - 2.0 * c[t] + ym) * xr.ih2 + am * zm[t] -
                                   (am + ap) * c[t] + ap * zp[t];
-                const double r = fv - lp;
-                if (in) {
-                    sr += r * r;
-                    sf += fv * fv;
-                    sx += c[t];
-                    if constexpr (STORE) st_stream(rrow + (size_t)t * w_tile<float>(), (float)r);
-                }
+                const double r = fv[t] - lp;
+                if constexpr (STORE) rs[t] = (float)r;
+                const double rm = act ? r : 0.0, fm = act ? fv[t] : 0.0, cm = act ? c[t] : 0.0;
+                sr += rm * rm;
+                sf += fm * fm;
+                sx += cm;
+            }
+            // the sums and r before the next loads (nothing below needs them,
+            // so the compiler would hold this plane's operands instead)
+            asm volatile("" : "+v"(sr), "+v"(sf), "+v"(sx));
+            if constexpr (STORE) {
+#pragma unroll
+                for (int t = 0; t < TY; ++t) asm volatile("" : "+v"(rs[t]));
             }
 #pragma unroll
             for (int t = 0; t < TY; ++t) {
                 zm[t] = c[t];
                 c[t] = zp[t];
+            }
+            pp += pl;
+            fp += (long)n2m * n1m;
+            if (k + 1 < k1) load();
+            if constexpr (STORE) {
+                if (act) {
+#pragma unroll
+                    for (int t = 0; t < TY; ++t) st_stream(rrow + t * w_tile<float>() + ru, rs[t]);
+                }
+                rrow += (size_t)xr.Ly * (size_t)xr.Lxs;
             }
         }
     }
@@ -1533,35 +1566,44 @@ k_residual(const double *__restrict__ f, XRes xr, int n1m, int n2m, int n3m, con
     }
 }
 
-// Planes per residual tile, and the tile count for TY rows per tile.
-constexpr int kResKZ = 32;
-inline long residual_tiles(int n1m, int n2m, int n3m, int ty) {
-    return (long)((n1m + 255) / 256) * (n2m / ty) * ((n3m + kResKZ - 1) / kResKZ);
+// Rows and planes of a residual tile and the workgroups of its launch (at most
+// most, one partial triple each).  Blocks of 8 rows and 32 planes read the
+// fewest halo cells; where they leave fewer than 16 waves per CU a problem is
+// cut into fewer planes and rows: 112 x 96 x 130 34.5 -> 15 us with the store
+// and 25.6 -> 12 without (one row and 32 planes a tile, 256 lanes on a row of
+// 112 cells before), 320 x 224 x 200 58.
+struct ResShape {
+    int ty, kz;
+    unsigned grid;
+};
+inline ResShape residual_shape(int n1m, int n2m, int n3m, int cus, int most) {
+    static const int shapes[][2] = {{8, 32}, {8, 16}, {4, 16}, {4, 8}, {2, 8}, {2, 4}};
+    ResShape q{};
+    long waves = 0;
+    for (const auto &v : shapes) {
+        if (n2m % v[0]) continue;
+        q.ty = v[0];
+        q.kz = v[1];
+        waves = (long)((n1m + 63) / 64) * (n2m / q.ty) * ((n3m + q.kz - 1) / q.kz);
+        if (waves >= 16L * cus) break;
+    }
+    q.grid = (unsigned)std::min<long>(std::min<long>(most, 8L * cus), (waves + 3) / 4);
+    return q;
 }
-// Rows per residual tile: the largest of 8, 4, 2 dividing n2m that still
-// leaves min_tiles tiles (small problems need the parallelism more than the
-// halo saving), else 1.
-inline int residual_rows(int n1m, int n2m, int n3m, long min_tiles) {
-    for (int ty = 8; ty > 1; ty >>= 1)
-        if (n2m % ty == 0 && residual_tiles(n1m, n2m, n3m, ty) >= min_tiles) return ty;
-    return 1;
-}
-// The launch (grid g <= tiles, one partial triple per workgroup).
 template <bool STORE>
-inline void launch_k_residual_s(int ty, int g, hipStream_t s, const double *f, const XRes &xr, int n1m, int n2m,
+inline void launch_k_residual_s(const ResShape &q, hipStream_t s, const double *f, const XRes &xr, int n1m, int n2m,
                                 int n3m, const int *gate) {
-    switch (ty) {
-        case 8: hipLaunchKernelGGL((k_residual<kResKZ, 8, STORE>), dim3(g), dim3(256), 0, s, f, xr, n1m, n2m, n3m, gate); break;
-        case 4: hipLaunchKernelGGL((k_residual<kResKZ, 4, STORE>), dim3(g), dim3(256), 0, s, f, xr, n1m, n2m, n3m, gate); break;
-        case 2: hipLaunchKernelGGL((k_residual<kResKZ, 2, STORE>), dim3(g), dim3(256), 0, s, f, xr, n1m, n2m, n3m, gate); break;
-        default: hipLaunchKernelGGL((k_residual<kResKZ, 1, STORE>), dim3(g), dim3(256), 0, s, f, xr, n1m, n2m, n3m, gate); break;
+    switch (q.ty) {
+        case 8: hipLaunchKernelGGL((k_residual<8, STORE>), dim3(q.grid), dim3(256), 0, s, f, xr, n1m, n2m, n3m, q.kz, gate); break;
+        case 4: hipLaunchKernelGGL((k_residual<4, STORE>), dim3(q.grid), dim3(256), 0, s, f, xr, n1m, n2m, n3m, q.kz, gate); break;
+        default: hipLaunchKernelGGL((k_residual<2, STORE>), dim3(q.grid), dim3(256), 0, s, f, xr, n1m, n2m, n3m, q.kz, gate); break;
     }
 }
 // r is stored (FP32, into xr.rout) when xr.rout is set
-inline void launch_k_residual(int ty, int g, hipStream_t s, const double *f, const XRes &xr, int n1m, int n2m, int n3m,
+inline void launch_k_residual(const ResShape &q, hipStream_t s, const double *f, const XRes &xr, int n1m, int n2m, int n3m,
                               const int *gate) {
-    if (xr.rout) launch_k_residual_s<true>(ty, g, s, f, xr, n1m, n2m, n3m, gate);
-    else launch_k_residual_s<false>(ty, g, s, f, xr, n1m, n2m, n3m, gate);
+    if (xr.rout) launch_k_residual_s<true>(q, s, f, xr, n1m, n2m, n3m, gate);
+    else launch_k_residual_s<false>(q, s, f, xr, n1m, n2m, n3m, gate);
 }
 
 }  // namespace ppf

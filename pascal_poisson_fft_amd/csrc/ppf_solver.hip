@@ -218,9 +218,10 @@ static XRes make_xres(const ppf_plan *p, const double *P) {
 // r is also stored in W32, where the refinement form of pass 1 reads it.
 // reduce = false skips the totals (a store right after a test of the same P,
 // whose totals are already in p->red); test folds the device-side
-// refinement test into the reduction.
+// refinement test into the reduction; host (pinned memory): the totals go
+// there too, for a caller that synchronises and reads them.
 static int launch_residual(ppf_plan *p, const double *f, const double *P, hipStream_t s, bool out = false,
-                           bool reduce = true, const GateTest &test = GateTest{}) {
+                           bool reduce = true, const GateTest &test = GateTest{}, double *host = nullptr) {
     const int n3m = p->d.n3m;
     XRes xr = make_xres(p, P);
     if (out) {
@@ -228,29 +229,23 @@ static int launch_residual(ppf_plan *p, const double *f, const double *P, hipStr
         xr.Ly = p->Ly;
         xr.Lxs = p->Lxs;
     }
-    const int ty = residual_rows(p->d.n1m, p->d.n2m, n3m, 4L * num_cus());
-    const long ntiles = residual_tiles(p->d.n1m, p->d.n2m, n3m, ty);
-    const int g = (int)std::min<long>(std::min<long>(p->npartial, 8L * num_cus()), ntiles);
-    launch_k_residual(ty, g, s, f, xr, p->d.n1m, p->d.n2m, n3m, p->gate);
-    if (reduce) hipLaunchKernelGGL(k_reduce3, dim3(1), dim3(256), 0, s, p->partial, g, p->red, p->gate, test);
+    const ResShape q = residual_shape(p->d.n1m, p->d.n2m, n3m, num_cus(), p->npartial);
+    launch_k_residual(q, s, f, xr, p->d.n1m, p->d.n2m, n3m, p->gate);
+    if (reduce)
+        hipLaunchKernelGGL(k_reduce3, dim3(1), dim3(256), 0, s, p->partial, (int)q.grid, p->red, p->gate, test, host);
     PPF_HIP(hipGetLastError());
     return PPF_OK;
 }
 
-// Ghost layers of P re-derived from its interior, in the reference's order
-// (walls x, y, z, then wraps x, y, z; fft_3d_poisson.f90:620-622).
+// Ghost layers of P re-derived from its interior.
 static int refresh_ghosts(const ppf_plan *p, double *P, const double *dmx1, const double *dmx2, const double *dmx3,
                           hipStream_t s) {
-    const int n[3] = {p->d.n1m, p->d.n2m, p->d.n3m};
-    const int per[3] = {p->d.pbc1 != 0, p->d.pbc2 != 0, p->d.pbc3 != 0};
-    const double *dmx[3] = {dmx1, dmx2, dmx3};
-    for (int wrap = 0; wrap < 2; ++wrap)
-        for (int dir = 0; dir < 3; ++dir) {
-            if (per[dir] != wrap) continue;
-            const size_t nb = (size_t)(dir == 0 ? n[1] : n[0]) + 2, nc = (size_t)(dir == 2 ? n[1] : n[2]) + 2;
-            const unsigned grid = (unsigned)((nb * nc + 255) / 256);
-            hipLaunchKernelGGL(k_ghost_face, dim3(grid), dim3(256), 0, s, P, n[0], n[1], n[2], dir, wrap, dmx[dir]);
-        }
+    const GhostArgs g{{p->d.n1m, p->d.n2m, p->d.n3m},
+                      {p->d.pbc1 != 0, p->d.pbc2 != 0, p->d.pbc3 != 0},
+                      {dmx1, dmx2, dmx3}};
+    const size_t n1 = p->d.n1m, n2 = p->d.n2m, n3 = p->d.n3m;
+    const size_t cells = 2 * ((n1 + 2) * (n2 + 2) + (n1 + 2) * n3 + n2 * n3);
+    hipLaunchKernelGGL(k_ghosts, dim3((unsigned)((cells + 255) / 256)), dim3(256), 0, s, P, g);
     PPF_HIP(hipGetLastError());
     return PPF_OK;
 }
@@ -305,8 +300,7 @@ static int solve_fp32_ir(ppf_plan *p, const double *f, double *P, const double *
         // 0.49 ms at 512^3) and a miss recomputes r with the store.
         for (;;) {
             const bool store = sweeps == 0 && sweeps < maxs;
-            if ((rc = launch_residual(p, f, P, s, store))) return rc;
-            PPF_HIP(hipMemcpyAsync(p->hred, p->red, 3 * sizeof(double), hipMemcpyDeviceToHost, s));
+            if ((rc = launch_residual(p, f, P, s, store, true, GateTest{}, p->hred))) return rc;
             PPF_HIP(hipStreamSynchronize(s));
             rel = p->hred[1] > 0 ? std::sqrt(p->hred[0] / p->hred[1]) : std::sqrt(p->hred[0]);
             if (rel <= tol) { converged = true; break; }
@@ -560,8 +554,7 @@ int ppf_residual(ppf_plan *p, const double *f, const double *P, const double *dm
     const int n3m = p->d.n3m;
     hipLaunchKernelGGL(k_zcoef, dim3((n3m + 255) / 256), dim3(256), 0, s, dx3, dmx3, n3m, p->zcoef, p->zcoef + n3m);
     int rc;
-    if ((rc = launch_residual(p, f, P, s))) return rc;
-    PPF_HIP(hipMemcpyAsync(p->hred, p->red, 3 * sizeof(double), hipMemcpyDeviceToHost, s));
+    if ((rc = launch_residual(p, f, P, s, false, true, GateTest{}, p->hred))) return rc;
     PPF_HIP(hipStreamSynchronize(s));
     *rel = p->hred[1] > 0 ? std::sqrt(p->hred[0] / p->hred[1]) : std::sqrt(p->hred[0]);
     return PPF_OK;
