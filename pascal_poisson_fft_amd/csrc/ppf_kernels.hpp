@@ -1110,24 +1110,17 @@ k_zthomas(T *__restrict__ W, T *__restrict__ cs, ZArgs z, const double *__restri
 // equation.  With x_0 and x_{K-1} known, a Thomas sweep over rows 1..K-2 that
 // reuses the forward multipliers C_l recovers the interior.  Both reduction
 // sweeps carry O(1) state, so a thread holds 2K values (its right-hand sides
-// and C).  Rows past n3m are identity rows.  Coefficients, pin, ghost planes
-// and mean as in k_zthomas.
+// and C).  Coefficients, pin, ghost planes and mean as in k_zthomas.
 // ---------------------------------------------------------------------------
-#ifndef PPF_RCP_NEWTON
-#define PPF_RCP_NEWTON 2
-#endif
 // FP32: the hardware reciprocal is correct to about 1 ulp
 __device__ __forceinline__ float frcp(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ double frcp(double x) {
-    // reciprocal: hardware estimate refined by Newton steps (each doubles the
-    // correct bits; two give about 1 ulp)
-    double r = __builtin_amdgcn_rcp(x);
-#pragma unroll
-    for (int i = 0; i < PPF_RCP_NEWTON; ++i) {
-        const double e = __builtin_fma(-x, r, 1.0);
-        r = __builtin_fma(r, e, r);
-    }
-    return r;
+    // reciprocal: hardware estimate r with x r = 1 - e, |e| about 2^-23, times
+    // 1 + e + e^2 (the rest, e^3, is below 2^-53): one operation and one link of
+    // the chain less than two Newton steps, as accurate
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = __builtin_fma(-x, r, 1.0);
+    return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 
 // WPE: minimum waves per SIMD the register allocation must allow (occupancy
@@ -1137,14 +1130,12 @@ __device__ __forceinline__ double frcp(double x) {
 //
 // Registers bound this kernel: 2K values a thread are the algorithm's own, and
 // what it holds beside them decides how many workgroups share a CU.  Row
-// addresses are therefore formed from one base at each access, masks are
-// comparisons with one row count, a row's coefficients are one 16-byte LDS
-// read, and every step of a sweep is pinned in its place: the empty volatile
-// asm of zp_pin takes the step's state and the LDS index, so neither is the
-// arithmetic moved behind the reads of all the later steps (the compiler
-// otherwise reads the coefficients of the whole sweep first) nor are the
-// coefficients and addresses of one sweep carried to the next.
-__device__ __forceinline__ void zp_pin(int &i) { asm volatile("" : "+v"(i)); }
+// addresses are therefore formed from one base at each access, a row's
+// coefficients are one 16-byte LDS read, and every step of a sweep is pinned in
+// its place: the empty volatile asm of zp_pin takes the step's state and the
+// LDS index, so neither is the arithmetic moved behind the reads of all the
+// later steps (the compiler otherwise reads the coefficients of the whole
+// sweep first) nor are the coefficients of one sweep carried to the next.
 __device__ __forceinline__ void zp_pin(int &i, double &a) { asm volatile("" : "+v"(i), "+v"(a)); }
 __device__ __forceinline__ void zp_pin(int &i, double &a, double &b) { asm volatile("" : "+v"(i), "+v"(a), "+v"(b)); }
 // LDS row of partition p: K coefficient pairs and one pad pair, so that the
@@ -1166,7 +1157,7 @@ k_zpart(T *__restrict__ W, ZArgs z, const double *__restrict__ zam, const double
     const int n3m = z.n3m;
     constexpr int KS = (K + S - 1) / S;           // table rows per thread
     const int NPAD = KS * (int)blockDim.x;        // >= P * K: every thread writes KS entries
-    D2 *co = reinterpret_cast<D2 *>(zsh);         // (am, ap) of row g at g + g / K; zero past n3m
+    D2 *co = reinterpret_cast<D2 *>(zsh);         // (am, ap) of row g at g + g / K; (0, 1) past n3m
     const int PS = P * S;
     CT *ra = reinterpret_cast<CT *>(co + zp_coef_slots<K>(NPAD));  // [3][P][S]: first-row equations, then reduction buffer
     CT *rc = ra + 3 * PS;           // [3][P][S]: reduction buffer
@@ -1194,8 +1185,8 @@ k_zpart(T *__restrict__ W, ZArgs z, const double *__restrict__ zam, const double
         return reinterpret_cast<T *>(reinterpret_cast<char *>(wl) + (size_t)(unsigned)l * (unsigned)rbytes);
     };
     const CT lx = (CT)z.lamx[kc0], ly = (CT)z.lamy[jp];
-    const int pin0 = (active & (z.zx[kc0] != 0) & (z.zy[jp] != 0) & (p == 0)) ? 0 : -1;  // row pinned in this partition
-    int nv = active ? n3m - g0 : 0;  // rows l < nv are real
+    const bool pin = active & (z.zx[kc0] != 0) & (z.zy[jp] != 0) & (p == 0);  // row 0 is pinned
+    const int nv = n3m - g0;  // rows l < nv are real
     // Row coefficients (the per-solve table filled by pass 1) are loaded
     // first: loads complete in order, so waiting for them does not wait for
     // the line loads issued after them.  Their LDS writes are unconditional
@@ -1220,55 +1211,57 @@ k_zpart(T *__restrict__ W, ZArgs z, const double *__restrict__ zam, const double
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
         const int k = tid + j * (int)blockDim.x;
-        co[k + k / K] = k < n3m ? D2{ca[j], cp[j]} : D2{0.0, 0.0};
+        co[k + k / K] = k < n3m ? D2{ca[j], cp[j]} : D2{0.0, 1.0};
     }
     __syncthreads();
-    // a row's value is masked where it is first used: zero past n3m, in
-    // inactive columns, and in the pinned first row of the (0,0) mode
-    CT d[K];
-    auto dmask = [&](int l) { d[l] = (l < nv && l != pin0) ? (CT)raw[l] : CT(0); };
-    // identity rows: padding past n3m, and the pinned first row of the (0,0) mode
-    int co0 = p * (K + 1);
-    auto coef = [&](int l, D2 ac, CT &a, CT &b, CT &c) {
-        const bool id = l >= nv || l == pin0;
-        a = (CT)ac.x;
-        c = id ? CT(0) : (CT)ac.y;
-        b = id ? CT(1) : (-(CT)ac.x - (CT)ac.y - lx) - ly;
-    };
-    // Reverse sweep (first-row equation) and forward sweep (last-row
-    // equation) interleaved: two independent dependency chains per step.
-    // The forward pivots r_l are kept for the final pass.  A step reads the
-    // next one's coefficients before its own arithmetic, so the LDS latency is
-    // not in the chain.
-    CT rr[K];
+    // Rows past n3m need no masks: the last real row has c = 0, so what they
+    // hold reaches no real row as long as it is finite, and the table gives
+    // them a regular diagonal for every mode.  Columns past Lx are copies that
+    // are not stored.  That leaves the pinned first row of the (0,0) mode, met
+    // once.  (Selects on every coefficient and value of every row were a third
+    // of this kernel's instructions: 1024 x 1024 x 768 2.92 -> 2.61 ms, 512^3 409
+    // -> 398 us, FP32 with 32 columns 430 -> 345, 320 x 224 x 200 63 -> 57.)
+    CT d[K], rr[K];
     CT ah, ch, dh, Af, Df, Cf;
+    int co0 = p * (K + 1);
     {
-        CT a, b, c;
-        dmask(K - 2);
-        dmask(1);
-        coef(K - 2, co[co0 + K - 2], a, b, c);
-        CT r = frcp(b);
-        ah = r * a; ch = r * c; dh = r * d[K - 2];
-        coef(1, co[co0 + 1], a, b, c);
-        r = frcp(b);
+        // Reverse sweep (first-row equation) and forward sweep (last-row
+        // equation) interleaved: two independent dependency chains per step.
+        // The forward pivots r_l are kept for the final pass.  A step reads
+        // the next one's coefficients before its own arithmetic, so the LDS
+        // latency is not in the chain.
+        // in the order of k_zthomas: where the rows are much finer than x and y,
+        // the rounding of this sum is most of a line's error, and lx + ly taken
+        // first gives another one (8e-11 instead of 2e-12 away at 3072 rows)
+        auto diag = [&](D2 ac) { return (-(CT)ac.x - (CT)ac.y - lx) - ly; };
+        D2 nb = co[co0 + K - 2], nf = co[co0 + 1];
+        d[K - 2] = (CT)raw[K - 2];
+        d[1] = (CT)raw[1];
+        CT r = frcp(diag(nb));
+        ah = r * (CT)nb.x; ch = r * (CT)nb.y; dh = r * d[K - 2];
+        r = frcp(diag(nf));
         rr[1] = r;
-        Af = r * a; Cf = r * c; Df = r * d[1];
-        D2 nb = co[co0 + K - 3], nf = co[co0 + 2];
+        Af = r * (CT)nf.x; Cf = r * (CT)nf.y; Df = r * d[1];
+        nb = co[co0 + K - 3];
+        nf = co[co0 + 2];
 #pragma unroll
         for (int i = 1; i <= K - 2; ++i) {
             const int lb = K - 2 - i;  // reverse row
             const int lf = 1 + i;      // forward row
-            const D2 cb = nb, cf = nf;
+            const CT a1 = (CT)nb.x, a2 = (CT)nf.x, c2 = (CT)nf.y, b2 = diag(nf);
+            CT c1 = (CT)nb.y, b1 = diag(nb);
             if (i < K - 2) {
                 nb = co[co0 + lb - 1];
                 nf = co[co0 + lf + 1];
             }
-            // a row is masked by the sweep that meets it first
-            if (2 * lb > K - 1 || lb == 0) dmask(lb);
-            if (2 * lf < K - 1 || lf == K - 1) dmask(lf);
-            CT a1, b1, c1, a2, b2, c2;
-            coef(lb, cb, a1, b1, c1);
-            coef(lf, cf, a2, b2, c2);
+            // a row's value is taken up by the sweep that meets it first
+            if (2 * lb > K - 1 || lb == 0) d[lb] = (CT)raw[lb];
+            if (2 * lf < K - 1 || lf == K - 1) d[lf] = (CT)raw[lf];
+            if (lb == 0) {
+                b1 = pin ? CT(1) : b1;
+                c1 = pin ? CT(0) : c1;
+                d[0] = pin ? CT(0) : d[0];
+            }
             const CT r1 = frcp(b1 - c1 * ah);
             const CT r2 = frcp(b2 - a2 * Cf);
             ch = -r1 * c1 * ch;
@@ -1279,7 +1272,7 @@ k_zpart(T *__restrict__ W, ZArgs z, const double *__restrict__ zam, const double
             Cf = r2 * c2;
             Df = r2 * (d[lf] - a2 * Df);
             zp_pin(co0, dh, Df);
-            zp_pin(nv, ch, Af);
+            zp_pin(co0, ch, Af);
         }
     }
     // Reduced system in the partition end values e_p = x_{K-1} of partition p.
@@ -1352,27 +1345,33 @@ k_zpart(T *__restrict__ W, ZArgs z, const double *__restrict__ zam, const double
             d[l] = e;
             zp_pin(co0, e);
         }
-        zp_pin(nv);
         x[0] = x0;
         x[K - 1] = xl;
         CT nc = (CT)co[co0 + K - 2].y;
 #pragma unroll
         for (int l = K - 2; l >= 1; --l) {
-            const CT c = (l >= nv || l == pin0) ? CT(0) : nc;
+            const CT c = nc;
             nc = (CT)co[co0 + l - 1].y;
             x[l] = d[l] - rr[l] * c * x[l + 1];
             zp_pin(co0, x[l]);
-            zp_pin(nv);
         }
     }
     asm volatile("" : "+s"(rbytes));
-    zp_pin(nv);
     CT xt = 0, xb = 0;  // the line's last two rows, in the partition that ends it (l = nv - 1)
+    if (active) {
+        if (nv >= K) {
 #pragma unroll
-    for (int l = 0; l < K; ++l) {
-        if (l < nv) st_stream(row(l), (T)x[l]);
-        xt = l == nv - 1 ? x[l] : xt;
-        xb = l == nv - 2 ? x[l] : xb;
+            for (int l = 0; l < K; ++l) st_stream(row(l), (T)x[l]);
+            xt = x[K - 1];
+            xb = x[K - 2];
+        } else {
+#pragma unroll
+            for (int l = 0; l < K; ++l) {
+                if (l < nv) st_stream(row(l), (T)x[l]);
+                xt = l == nv - 1 ? x[l] : xt;
+                xb = l == nv - 2 ? x[l] : xb;
+            }
+        }
     }
     // spectral z ghost planes: wall extrapolation (fft_3d_poisson.f90:809-852)
     // or, for periodic z, the wrapped end planes (:666-796)

@@ -14,24 +14,25 @@ constexpr int kZLong8 = 18, kZLong4 = 19;
 // unless another grid is named, this rule's shape against the neighbours:
 //  * up to 512 rows, about 16 partitions: S P then fills whole groups of four
 //    waves, one for each SIMD (a six-wave workgroup of 28 or 32 rows gets one
-//    place where two would fit): 300 rows K=20 104, K=32 111, K=16 124;
-//    384 rows K=24 117, 32 122, 16 135; 448 rows K=28 127, 32 137, 16 145;
-//    200 rows K=20 66, K=16 69, K=32 73;
+//    place where two would fit): 300 rows K=20 102, K=32 107, K=16 117;
+//    448 rows K=28 127, 32 141, 16 147; 200 rows K=20 54, K=16 57, K=32 60;
 //  * 513..768 rows K = 24, whose 128 registers admit two 512-thread
-//    workgroups per CU: 768 rows 266, K=28 319, K=32 348 (1024 x 1024 x 768:
-//    2.92 ms, K=32 4.31 ms);
-//  * FP32 workspaces up to 256 rows take 32 columns, whole 128-byte rows:
-//    256 rows (32,32) 46, (16,16) 59; 128 rows (16,32) 26, (8,16) 29;
+//    workgroups per CU: 768 rows 253, K=28 294, K=32 310 (1024 x 1024 x 768:
+//    2.61 ms, K=32 3.90 ms);
+//  * FP32 workspaces up to 256 and near 512 rows take 32 columns, whole
+//    128-byte rows: 256 rows (32,32) 44, (16,16) 58; 128 rows (16,32) 22,
+//    (8,16) 28; 512 rows (32,32) 109, (32,16) 135 (512^3: 345, 405); 384 rows
+//    (32,32) 90, (24,16) 81;
 //  * fewer workgroups than four per CU (they are all resident at once, so a
 //    line's chain of rows is what counts): 8 columns and short partitions.
-//    64 x 64 lines (PP) of 64 rows: (8,8) 8.4, (16,16) 10.0, (32,16) 13.1; of
-//    512 rows (16,8) 16.1, (8,8) 18.9, (32,16) 19.6; of 768 rows (24,8) 20.8,
-//    (24,16) 25.8; of 1024 rows (32,8) 26.0, (32,16) 39.7;
+//    64 x 64 lines (PP) of 64 rows: (8,8) 7.7, (16,16) 8.5, (32,16) 10.5; of
+//    512 rows (16,8) 14.7, (8,8) 17.0, (32,16) 15.9; of 768 rows (24,8) 20,
+//    (24,16) 21, (32,16) 29; of 1024 rows (32,8) 28, (32,16) 34;
 //  * over 1024 rows 8 columns (a 16-column workgroup exceeds 512 threads or
 //    its registers) and K = 48; 1537..2048 rows K = 32.  128 x 128 lines of
-//    1536 rows K=48 145, 32 186; of 2048 rows K=32 222, 48 249; of 2050 rows
-//    K=48 253, one thread per line 1829; of 4096 rows (K = 48, 4 columns)
-//    1081, one thread per line 3820.
+//    1536 rows K=48 128, 32 164; of 2048 rows K=32 201, 48 220; of 2050 rows
+//    K=48 219, one thread per line 1822; of 4096 rows (K = 48, 4 columns)
+//    948, one thread per line 3823.
 template <typename T>
 int z_default(int n3m, int nwg16) {
     if (n3m > 2048) return n3m <= 3072 ? kZLong8 : kZLong4;
@@ -39,6 +40,7 @@ int z_default(int n3m, int nwg16) {
     if (nwg16 < 4 * num_cus()) return n3m <= 400 ? 5 : (n3m <= 512 ? 2 : (n3m <= 768 ? 13 : 4));
     if (n3m <= 24) return 11;
     if (sizeof(T) == 4 && n3m <= 256) return n3m <= 128 ? 16 : 15;
+    if (sizeof(T) == 4 && n3m > 416 && n3m <= 512) return 15;
     if (n3m <= 64) return 1;
     if (n3m <= 128) return 11;
     if (n3m <= 320) return 7;

@@ -21,7 +21,7 @@ from pascal_poisson_fft_amd.grid import make_axis
 pytestmark = pytest.mark.gpu
 
 SMALL = [8, 24, 26, 400, 402, 512, 514, 768, 770, 1024, 1026, 1536, 1538, 2048, 2050, 3072, 3074, 4096]
-LARGE = [4, 24, 26, 64, 66, 128, 130, 256, 258, 320, 322, 384, 386, 448, 450, 512, 514, 768, 770, 1022]
+LARGE = [4, 24, 26, 64, 66, 128, 130, 256, 258, 320, 322, 384, 386, 416, 418, 448, 450, 512, 514, 768, 770, 1022]
 
 
 def _solve(n1, n2, n3, pbc, precision):
