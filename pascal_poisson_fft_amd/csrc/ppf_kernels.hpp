@@ -1011,82 +1011,241 @@ struct ZArgs {
     const int *gate;                  // refinement gate (gated_off), nullptr = always run
 };
 
+// FP32: the hardware reciprocal is correct to about 1 ulp
+__device__ __forceinline__ float frcp(float x) { return __builtin_amdgcn_rcpf(x); }
+__device__ __forceinline__ double frcp(double x) {
+    // reciprocal: hardware estimate r with x r = 1 - e, |e| about 2^-23, times
+    // 1 + e + e^2 (the rest, e^3, is below 2^-53): one operation and one link of
+    // the chain less than two Newton steps, as accurate
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = __builtin_fma(-x, r, 1.0);
+    return __builtin_fma(r, __builtin_fma(e, e, e), r);
+}
+
+// This kernel is bound by a line's chain of rows and by what its one wave can
+// issue (0.12 us a row both ways), once nothing else is waited for:
+//  * rows come in chunks of kZtRows, the next chunk's loads in flight while the
+//    current one is solved;
+//  * a wave may have 63 memory operations in flight and a row takes three, so
+//    one operation moves two rows of 32 lines (a half of the wave each); a lane
+//    swap hands both rows to both halves, which run the same chain;
+//  * a chunk's coefficients are one load of the wave, a row to a lane, handed
+//    out by lane reads: scalar loads return out of order, so each would be
+//    waited for where it is used;
+//  * one-wave workgroups spread few lines over as many CUs.
+// z stage, 256-thread workgroups with each row's loads where they are used ->
+// this form, the same bits: 96 x 80 lines of 2050 rows 1589 -> 277 us, 128 x
+// 128 1804 -> 355, 256 x 256 of 2052 2533 -> 1356, 64 x 64 of 512 401 -> 73.
+// One row of 64 lines an operation: 302, 335, 1270, 81; four of 16: 291, 456,
+// 1362, 77.  (The partitioned form of k_zpart takes 130 us on the first of
+// these, but adds up to 1.6e-11 to lines this long, which is more than FP64
+// solves are held to.)
+constexpr int kZtRows = 32;
+
+__device__ __forceinline__ double lane_read(double v, int lane) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, lane);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), lane);
+    return __builtin_bit_cast(double, (unsigned long long)lo | (unsigned long long)hi << 32);
+}
+
+// x[h] = v of wave half h, in both halves
+__device__ __forceinline__ void zt_spread(unsigned v, unsigned (&x)[2]) {
+    const auto q = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    x[0] = q[0];
+    x[1] = q[1];
+}
+__device__ __forceinline__ void zt_spread(float v, double (&x)[2]) {
+    unsigned u[2];
+    zt_spread(__builtin_bit_cast(unsigned, v), u);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) x[h] = (double)__builtin_bit_cast(float, u[h]);
+}
+__device__ __forceinline__ void zt_spread(double v, double (&x)[2]) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    unsigned lo[2], hi[2];
+    zt_spread((unsigned)b, lo);
+    zt_spread((unsigned)(b >> 32), hi);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        x[h] = __builtin_bit_cast(double, (unsigned long long)lo[h] | (unsigned long long)hi[h] << 32);
+}
+
+// The lane's view of an array: row k + h of its line, h the wave half, at byte
+// k * pitch + off (off holds h rows).  The row part stays in scalar registers,
+// advanced two rows at a time.
 template <typename T>
-__global__ void __launch_bounds__(256)
-k_zthomas(T *__restrict__ W, T *__restrict__ cs, ZArgs z, const double *__restrict__ dx3,
-          const double *__restrict__ dmx3, double *__restrict__ mean_out) {
+struct ZLines {
+    T *base;
+    size_t pitch;
+    unsigned off;
+    __device__ __forceinline__ T &at(size_t row) const {
+        return *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + row + off);
+    }
+    // rows k0 .. k0 + kZtRows - 1 (k0 and n even); past the line its last two again
+    __device__ __forceinline__ void load(T (&v)[kZtRows / 2], int k0, int n) const {
+        size_t q = (size_t)k0 * pitch;
+        if (k0 + kZtRows <= n) {
+#pragma unroll
+            for (int i = 0; i < kZtRows / 2; ++i) {
+                v[i] = at(q);
+                q += 2 * pitch;
+                asm volatile("" : "+s"(q));
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < kZtRows / 2; ++i)
+                v[i] = at((size_t)(k0 + 2 * i + 2 <= n ? k0 + 2 * i : n - 2) * pitch);
+        }
+    }
+};
+
+template <typename T>
+__global__ void __launch_bounds__(64)
+k_zthomas(T *W, T *cs, ZArgs z, const double *__restrict__ zam, const double *__restrict__ zap,
+          double *__restrict__ mean_out) {
     if (gated_off(z.gate)) return;
-    extern __shared__ double zsh[];
-    double *am = zsh, *ap = zsh + z.n3m;
-    for (int k = threadIdx.x; k < z.n3m; k += blockDim.x) {
-        const int kk = k + 1;
-        double m = 1.0 / dx3[kk] / dmx3[kk];
-        double p = 1.0 / dx3[kk] / dmx3[kk + 1];
-        if (kk == 1) m = 0.0;
-        if (kk == z.n3m) p = 0.0;
-        am[k] = m;
-        ap[k] = p;
-    }
-    __syncthreads();
-    // wall extrapolation of cuda_neumann_BC (fft_3d_poisson.f90:829-837)
-    double bca0, bcb0, bca1, bcb1;
-    {
-        const double d1 = dmx3[1], d2 = dmx3[2], s0 = d1 + d2;
-        bca0 = s0 * s0 / (s0 * s0 - d1 * d1);
-        bcb0 = d1 * d1 / (s0 * s0 - d1 * d1);
-        const double e1 = dmx3[z.n3m + 1], e2 = dmx3[z.n3m], s1 = e1 + e2;
-        bca1 = s1 * s1 / (s1 * s1 - e1 * e1);
-        bcb1 = e1 * e1 / (s1 * s1 - e1 * e1);
-    }
-    const long col = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (col >= (long)z.Lx * z.njr) return;
-    const int kx = (int)(col % z.Lx);
-    const int jp = z.jlo + (int)(col / z.Lx);
+    constexpr int WT = w_tile<T>(), RJ = 32 / WT, U = kZtRows, G = U / 2;
+    const int tid = (int)threadIdx.x, half = tid / 32, ln = tid % 32;
+    const int tiles = (z.Lx + WT - 1) / WT;
+    const int kxt = (int)(blockIdx.x % (unsigned)tiles) * WT + ln % WT;
+    const int jrt = (int)(blockIdx.x / (unsigned)tiles) * RJ + ln / WT;
+    // a lane past the edges solves the last column or row again, which is a line
+    // of the same wave: it stores what that lane stores, in the same instruction
+    const int kx = kxt < z.Lx ? kxt : z.Lx - 1, jr = jrt < z.njr ? jrt : z.njr - 1;
+    const int jp = z.jlo + jr;
+    const int n = z.n3m;
     const size_t pstride = (size_t)z.Ly * z.Lxs;
-    T *w = W + w_at<T>(jp, kx, z.Ly);      // plane 0 of this column
-    T *c = cs + (size_t)(col);               // scratch, stride Lx*njr
-    const size_t cstride = (size_t)z.Lx * z.njr;
+    T *w = W + w_at<T>(jp, kx, z.Ly);  // plane 0 of this column
+    const size_t wp = pstride * sizeof(T), cp = (size_t)z.Lx * z.njr * sizeof(T);
+    const ZLines<T> wr{W + pstride, wp, (unsigned)(w_at<T>(jp, kx, z.Ly) * sizeof(T) + (size_t)half * wp)};
+    const ZLines<T> cr{cs, cp, (unsigned)(((size_t)jr * z.Lx + (size_t)kx) * sizeof(T) + (size_t)half * cp)};
     const double lx = z.lamx[kx], ly = z.lamy[jp];
     const bool pin = z.zx[kx] && z.zy[jp];
-    const int n = z.n3m;
+    double dprev = 0.0, cprev = 0.0;
     // forward elimination
-    double b1 = (-am[0] - ap[0] - lx) - ly;
-    double c1 = ap[0];
-    double d1 = (double)w[pstride];
-    if (pin) { b1 = 1.0; c1 = 0.0; d1 = 0.0; }
-    double dprev = d1 / b1;
-    double cprev = c1 / b1;
-    w[pstride] = (T)dprev;
-    c[0] = (T)cprev;
-    for (int k = 1; k < n; ++k) {
-        const double a = am[k], b = (-am[k] - ap[k] - lx) - ly, cc = ap[k];
-        const double d = (double)w[(size_t)(k + 1) * pstride];
-        const double r = 1.0 / (b - a * cprev);
-        dprev = r * (d - a * dprev);
-        cprev = r * cc;
-        w[(size_t)(k + 1) * pstride] = (T)dprev;
-        c[(size_t)k * cstride] = (T)cprev;
+    {
+        T cur[G], nxt[G];
+        double ca, cb, na = 0.0, nb = 0.0;  // coefficients of row k0 + tid (tid < U)
+        auto coefs = [&](int k0, double &a, double &b) {
+            const int k = k0 + (tid & (U - 1)) < n ? k0 + (tid & (U - 1)) : n - 1;
+            a = zam[k];
+            b = zap[k];
+        };
+        // a row's diagonal is formed a step early, out of the chain
+        double ra, rc, rb;
+        auto ready = [&](int u) {
+            ra = lane_read(ca, u);
+            rc = lane_read(cb, u);
+            rb = (-ra - rc - lx) - ly;
+        };
+        coefs(0, ca, cb);
+        wr.load(cur, 0, n);
+        for (int k0 = 0; k0 < n; k0 += U) {
+            if (k0 + U < n) {
+                coefs(k0 + U, na, nb);
+                wr.load(nxt, k0 + U, n);
+            }
+            auto chunk = [&](auto whole) {
+                constexpr bool WHOLE = decltype(whole)::value;  // the line reaches past the chunk's rows
+                size_t wq = (size_t)k0 * wp, cq = (size_t)k0 * cp;
+                ready(0);
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    double d[2], od[2], oc[2];
+                    zt_spread(cur[g], d);
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const int u = 2 * g + q;
+                        if (WHOLE || k0 + u < n) {
+                            const double a = ra, cc = rc, pivot = rb - a * cprev;
+                            if (u + 1 < U) ready(u + 1);
+                            if (u == 0 && k0 == 0) {
+                                const double b1 = pin ? 1.0 : pivot;
+                                dprev = (pin ? 0.0 : d[0]) / b1;
+                                cprev = (pin ? 0.0 : cc) / b1;
+                            } else {
+                                const double rv = frcp(pivot);
+                                dprev = rv * (d[q] - a * dprev);
+                                cprev = rv * cc;
+                            }
+                        }
+                        od[q] = dprev;
+                        oc[q] = cprev;
+                    }
+                    if (WHOLE || k0 + 2 * g < n) {
+                        wr.at(wq) = (T)(half ? od[1] : od[0]);
+                        cr.at(cq) = (T)(half ? oc[1] : oc[0]);
+                    }
+                    wq += 2 * wp;
+                    cq += 2 * cp;
+                    asm volatile("" : "+s"(wq), "+s"(cq));
+                }
+            };
+            if (k0 + U <= n) chunk(std::true_type{});
+            else chunk(std::false_type{});
+#pragma unroll
+            for (int i = 0; i < G; ++i) cur[i] = nxt[i];
+            ca = na;
+            cb = nb;
+        }
     }
-    // back substitution
-    double xn = dprev, xk = xn, xk1 = 0.0;
-    double sum = xn;
-    for (int k = n - 2; k >= 0; --k) {
-        const double ck = (double)c[(size_t)k * cstride];
-        const double dk = (double)w[(size_t)(k + 1) * pstride];
-        xk1 = xk;
-        xk = dk - ck * xk1;
-        w[(size_t)(k + 1) * pstride] = (T)xk;
-        sum += xk;
+    // back substitution, chunks downwards; the first one holds rows n - 1 (done)
+    // and n - 2 (n is even)
+    const double xn = dprev;
+    double xk = xn, xk1 = 0.0, sum = xn, xm1 = 0.0;
+    {
+        T vc[G], vd[G], nc[G], nd[G];
+        int k0 = (n - 1) / U * U;
+        cr.load(vc, k0, n);
+        wr.load(vd, k0, n);
+        for (; k0 >= 0; k0 -= U) {
+            if (k0 > 0) {
+                cr.load(nc, k0 - U, n);
+                wr.load(nd, k0 - U, n);
+            }
+            auto chunk = [&](auto whole) {
+                constexpr bool WHOLE = decltype(whole)::value;  // no row past n - 2
+                size_t wq = (size_t)(k0 + U - 2) * wp;
+#pragma unroll
+                for (int g = G - 1; g >= 0; --g) {
+                    double c[2], d[2], x[2];
+                    zt_spread(vc[g], c);
+                    zt_spread(vd[g], d);
+#pragma unroll
+                    for (int q = 1; q >= 0; --q) {
+                        if (WHOLE || k0 + 2 * g + q <= n - 2) {
+                            xk1 = xk;
+                            xk = d[q] - c[q] * xk1;
+                            sum += xk;
+                        }
+                        if (!WHOLE && k0 + 2 * g + q == n - 2) xm1 = (double)(T)xk;
+                        x[q] = xk;
+                    }
+                    if (WHOLE || k0 + 2 * g + half <= n - 2) wr.at(wq) = (T)(half ? x[1] : x[0]);
+                    wq -= 2 * wp;
+                    asm volatile("" : "+s"(wq));
+                }
+            };
+            if (k0 + U <= n - 1) chunk(std::true_type{});
+            else chunk(std::false_type{});
+#pragma unroll
+            for (int i = 0; i < G; ++i) {
+                vc[i] = nc[i];
+                vd[i] = nd[i];
+            }
+        }
     }
-    // now xk = x_1, xk1 = x_2; x_n and x_{n-1} are re-read (n >= 2)
-    const double x1 = xk, x2 = xk1;
-    const double xm1 = (double)w[(size_t)(n - 1) * pstride];
+    if (half) return;
+    // now xk = x_1, xk1 = x_2, xm1 = x_{n-1} as it was stored
+    const double *bc = zap + n;  // wall extrapolation of cuda_neumann_BC (fft_3d_poisson.f90:829-837)
+    T *wn = w + (size_t)(n + 1) * pstride;
     if (z.zper) {
-        w[0] = (T)xn;
-        w[(size_t)(n + 1) * pstride] = (T)x1;
+        *w = (T)xn;
+        *wn = (T)xk;
     } else {
-        w[0] = (T)(bca0 * x1 - bcb0 * x2);
-        w[(size_t)(n + 1) * pstride] = (T)(bca1 * xn - bcb1 * xm1);
+        *w = (T)(bc[0] * xk - bc[1] * xk1);
+        *wn = (T)(bc[2] * xn - bc[3] * xm1);
     }
     if (kx == z.mean_kx && jp == z.mean_jp) *mean_out = sum * z.mean_scale;
 }
@@ -1112,17 +1271,6 @@ k_zthomas(T *__restrict__ W, T *__restrict__ cs, ZArgs z, const double *__restri
 // sweeps carry O(1) state, so a thread holds 2K values (its right-hand sides
 // and C).  Coefficients, pin, ghost planes and mean as in k_zthomas.
 // ---------------------------------------------------------------------------
-// FP32: the hardware reciprocal is correct to about 1 ulp
-__device__ __forceinline__ float frcp(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ double frcp(double x) {
-    // reciprocal: hardware estimate r with x r = 1 - e, |e| about 2^-23, times
-    // 1 + e + e^2 (the rest, e^3, is below 2^-53): one operation and one link of
-    // the chain less than two Newton steps, as accurate
-    const double r = __builtin_amdgcn_rcp(x);
-    const double e = __builtin_fma(-x, r, 1.0);
-    return __builtin_fma(r, __builtin_fma(e, e, e), r);
-}
-
 // WPE: minimum waves per SIMD the register allocation must allow (occupancy
 // is what lets one workgroup's loads overlap another's arithmetic here).
 // CT: arithmetic type (FP64 for every plan: FP32 arithmetic on FP32 storage

@@ -120,9 +120,13 @@ int ppf_plan_create(const ppf_desc *desc, ppf_plan **out) {
     plan_geometry(d, p);
     const bool fp32 = d.precision == PPF_PREC_FP32_IR;
     const size_t wsz = (size_t)p->Lxs * p->Ly * p->Lz;
-    // (the Thomas scratch cs is allocated by ppf_plan_set_zvariant, when the
-    // one-thread-per-line kernel is selected)
-    if ((rc = fp32 ? dev_alloc(p, &p->W32, wsz) : dev_alloc(p, &p->W, wsz)) || (rc = dev_alloc(p, &p->lamx, p->Lx)) ||
+    // Thomas scratch only where the one-thread-per-line kernel runs by
+    // default (n3m > 2048); ppf_plan_set_zvariant allocates it when that
+    // kernel is selected explicitly
+    const bool need_cs = d.n3m > 2048;
+    const size_t csz = need_cs ? (size_t)p->Lx * p->znjr * d.n3m : 1;
+    p->cs_elems = csz;
+    if ((rc = fp32 ? dev_alloc(p, &p->W32, wsz) : dev_alloc(p, &p->W, wsz)) || (rc = dev_alloc(p, &p->cs, csz)) || (rc = dev_alloc(p, &p->lamx, p->Lx)) ||
         (rc = dev_alloc(p, &p->lamy, p->Ly)) || (rc = dev_alloc(p, &p->zx, p->Lx)) || (rc = dev_alloc(p, &p->zy, p->Ly)) ||
         (rc = dev_alloc(p, &p->mean, 1)) || (rc = dev_alloc(p, &p->red, 3)) ||
         (rc = dev_alloc(p, &p->zcoef, 2 * (size_t)d.n3m + 4))) {
@@ -664,17 +668,16 @@ extern "C" int ppf_solve_noalloc(const ppf_desc *desc, const double *prhs, doubl
     const int Mx = (p.xkind == AX_C2C) ? desc->n1m : desc->n1m / 2;
     const int My = (p.ykind == AX_C2C) ? desc->n2m : desc->n2m / 2;
     const int n3m = desc->n3m;
-    // over 2048 rows the limit also counts one value per mode and row, which a
-    // one-thread-per-line z solve would keep
-    const bool long_z = n3m > 2048;
+    const bool need_cs = n3m > 2048;  // the one-thread-per-line z kernel's multipliers
     // bytes the slices below take (each rounded up to 256)
     auto sz = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
     const size_t need = sz(sizeof(double) * (size_t)p.Lxs * p.Ly * p.Lz) + sz(sizeof(cx<double>) * Mx) +
                         2 * sz(sizeof(cx<double>) * (Mx + 1)) + sz(sizeof(cx<double>) * My) +
                         2 * sz(sizeof(cx<double>) * (My + 1)) + sz(sizeof(double) * (2 * (size_t)n3m + 4)) +
                         sz(sizeof(double) * p.Lx) + sz(sizeof(double) * p.Ly) + sz(p.Lx) + sz(p.Ly) +
-                        sz(sizeof(double));
-    if (need + (long_z ? sz(sizeof(double) * (size_t)p.Lx * p.znjr * n3m) : 0) > kScratchBytes) return PPF_ERR_SCRATCH;
+                        sz(sizeof(double)) +
+                        (need_cs ? sz(sizeof(double) * (size_t)p.Lx * p.znjr * n3m) : 0);
+    if (need > kScratchBytes) return PPF_ERR_SCRATCH;
     double *base = nullptr;
     if ((rc = scratch_base(&base))) return rc;
     ScratchCarver c{reinterpret_cast<char *>(base)};
@@ -691,6 +694,10 @@ extern "C" int ppf_solve_noalloc(const ppf_desc *desc, const double *prhs, doubl
     p.zx = c.take<unsigned char>(p.Lx);
     p.zy = c.take<unsigned char>(p.Ly);
     p.mean = c.take<double>(1);
+    if (need_cs) {
+        p.cs_elems = (size_t)p.Lx * p.znjr * n3m;
+        p.cs = c.take<double>(p.cs_elems);
+    }
     if (c.used != need) return PPF_ERR_UNSUPPORTED;  // the size check and the slices disagree
     hipStream_t s = static_cast<hipStream_t>(stream);
     NoAllocTables t{};

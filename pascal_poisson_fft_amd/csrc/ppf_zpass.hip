@@ -8,7 +8,6 @@
 namespace ppf {
 
 namespace {
-constexpr int kZLong8 = 18, kZLong4 = 19;
 // The shape of a plan that was not tuned, from the line length and the number
 // of 16-column workgroups.  z stage in us, 256 x 256 lines (65536 columns)
 // unless another grid is named, this rule's shape against the neighbours:
@@ -30,12 +29,11 @@ constexpr int kZLong8 = 18, kZLong4 = 19;
 //    (24,16) 21, (32,16) 29; of 1024 rows (32,8) 28, (32,16) 34;
 //  * over 1024 rows 8 columns (a 16-column workgroup exceeds 512 threads or
 //    its registers) and K = 48; 1537..2048 rows K = 32.  128 x 128 lines of
-//    1536 rows K=48 128, 32 164; of 2048 rows K=32 201, 48 220; of 2050 rows
-//    K=48 219, one thread per line 1822; of 4096 rows (K = 48, 4 columns)
-//    948, one thread per line 3823.
+//    1536 rows K=48 128, 32 164; of 2048 rows K=32 201, 48 220;
+//  * longer lines one thread a line (k_zthomas, where the reason stands).
 template <typename T>
 int z_default(int n3m, int nwg16) {
-    if (n3m > 2048) return n3m <= 3072 ? kZLong8 : kZLong4;
+    if (n3m > 2048) return 6;
     if (n3m > 1024) return n3m <= 1536 ? 14 : 4;
     if (nwg16 < 4 * num_cus()) return n3m <= 400 ? 5 : (n3m <= 512 ? 2 : (n3m <= 768 ? 13 : 4));
     if (n3m <= 24) return 11;
@@ -73,14 +71,14 @@ int launch_z(ppf_plan *p, T *W, const double *dx3, const double *dmx3, hipStream
     const int n3m = p->d.n3m;
     // partitioned register-resident Thomas, shape (K rows per thread, S
     // columns per workgroup); launched only when S*P <= NTMAX, the LDS
-    // footprint stays within `lds` and n3m within `most`
+    // footprint stays within 64 KB and n3m within `most`
     bool done = false;
-    auto part = [&](auto kk, auto ss, auto nt, auto wpe, int most = 4096, size_t lds = 65536) {
+    auto part = [&](auto kk, auto ss, auto nt, auto wpe, int most = 4096) {
         constexpr int K = decltype(kk)::value, S = decltype(ss)::value;
         constexpr int NTMAX = decltype(nt)::value, WPE = decltype(wpe)::value;
         const int P = (n3m + K - 1) / K;
         const size_t shm = zp_lds_bytes<K, S>(P);
-        if (P < 1 || S * P > NTMAX || shm > lds || n3m > most) return;
+        if (P < 1 || S * P > NTMAX || shm > 65536 || n3m > most) return;
         const int tiles = (p->Lx + S - 1) / S;
         const int ntiles = tiles * p->znjr;
         // FP64 arithmetic for FP32 storage too: FP32 arithmetic measured no
@@ -111,9 +109,6 @@ int launch_z(ppf_plan *p, T *W, const double *dx3, const double *dmx3, hipStream
         case 15: part(PPF_Z(32, 32, 512, 3)); break;
         case 16: part(PPF_Z(16, 32, 512, 4)); break;
         case 17: part(PPF_Z(28, 16, 512, 3), 768); break;
-        // lines over 2048 rows (not selectable)
-        case kZLong8: part(PPF_Z(48, 8, 512, 2), 3072, 160 * 1024); break;
-        case kZLong4: part(PPF_Z(48, 4, 512, 2), 4096, 160 * 1024); break;
         default: break;
     }
 #undef PPF_Z
@@ -123,11 +118,10 @@ int launch_z(ppf_plan *p, T *W, const double *dx3, const double *dmx3, hipStream
         const long ncol = (long)p->Lx * p->znjr;
         // the one-thread-per-line kernel keeps its forward multipliers in cs
         if (p->cs_elems < (size_t)ncol * (size_t)n3m) return PPF_ERR_UNSUPPORTED;
-        const int nt = 256;
-        const size_t shm = 2 * sizeof(double) * (size_t)n3m;
-        hipLaunchKernelGGL((k_zthomas<T>), dim3((unsigned)((ncol + nt - 1) / nt)), dim3(nt), shm, s, W,
-                           reinterpret_cast<T *>(p->cs), z,
-                           dx3, dmx3, p->mean);
+        constexpr int wt = w_tile<T>(), rj = 32 / wt;
+        const unsigned blocks = (unsigned)((p->Lx + wt - 1) / wt) * (unsigned)((p->znjr + rj - 1) / rj);
+        hipLaunchKernelGGL((k_zthomas<T>), dim3(blocks), dim3(64), 0, s, W, reinterpret_cast<T *>(p->cs), z, p->zcoef,
+                           p->zcoef + n3m, p->mean);
     }
     return PPF_OK;
 }

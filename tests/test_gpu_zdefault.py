@@ -24,7 +24,7 @@ SMALL = [8, 24, 26, 400, 402, 512, 514, 768, 770, 1024, 1026, 1536, 1538, 2048, 
 LARGE = [4, 24, 26, 64, 66, 128, 130, 256, 258, 320, 322, 384, 386, 416, 418, 448, 450, 512, 514, 768, 770, 1022]
 
 
-def _solve(n1, n2, n3, pbc, precision):
+def _solve(n1, n2, n3, pbc, precision, zvariant=0):
     L = (2.0, 3.0, 1.5)
     ax, ay = make_axis(n1, L[0], pbc[0]), make_axis(n2, L[1], pbc[1])
     az = make_axis(n3, L[2], False, uniform=False, gamma=1.6)
@@ -32,6 +32,7 @@ def _solve(n1, n2, n3, pbc, precision):
     f -= float(np.einsum("kji,k->", f, az.dx[1:n3 + 1])) / (az.dx[1:n3 + 1].sum() * n1 * n2)
     ref = O.solve(f, L, (pbc[0], pbc[1], False), ax.dmx, ay.dmx, az.dmx, az.dx)
     plan = api.FFTPoisson(n1, n2, n3, L, (pbc[0], pbc[1], False), precision=precision)
+    plan.set_zvariant(zvariant)
     dev = api.Problem3D(f, ax, ay, az)
     try:
         args = (dev.rhs, dev.p, dev.dmx1, dev.dmx2, dev.dmx3, dev.dx3)
@@ -51,4 +52,14 @@ def test_default_z_shape_matches_oracle(n1, n2, n3, precision):
     pbc = (n3 % 4 == 2, n3 % 8 >= 4)
     err = _solve(n1, n2, n3, pbc, precision)
     bar = (1e-12 if n3 <= 512 else 1e-11) if precision == api.PPF_PREC_FP64 else 5e-6
+    assert err <= bar, err
+
+
+@pytest.mark.parametrize("precision", [api.PPF_PREC_FP64, api.PPF_PREC_FP32_IR], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("n3", [2, 4, 30, 32, 34, 62, 64, 66, 96, 130])
+def test_one_thread_per_line_matches_oracle(n3, precision):
+    """The one-thread-per-line solve around its 32-row chunks: lines within one
+    chunk, whole chunks, and one pair of rows past them; ragged columns."""
+    err = _solve(20, 12, n3, (n3 % 4 == 2, n3 % 8 >= 4), precision, zvariant=6)
+    bar = 1e-12 if precision == api.PPF_PREC_FP64 else 5e-6
     assert err <= bar, err
