@@ -27,14 +27,16 @@ namespace {
 //    64 x 64 lines (PP) of 64 rows: (8,8) 7.7, (16,16) 8.5, (32,16) 10.5; of
 //    512 rows (16,8) 14.7, (8,8) 17.0, (32,16) 15.9; of 768 rows (24,8) 20,
 //    (24,16) 21, (32,16) 29; of 1024 rows (32,8) 28, (32,16) 34;
-//  * over 1024 rows 8 columns (a 16-column workgroup exceeds 512 threads or
-//    its registers) and K = 48; 1537..2048 rows K = 32.  128 x 128 lines of
-//    1536 rows K=48 128, 32 164; of 2048 rows K=32 201, 48 220;
+//  * 1025..2048 rows 8 columns (a 16-column workgroup exceeds 512 threads or
+//    its registers) and K = 32: 128 x 128 lines of 2048 rows 201, K=48 220.
+//    K = 48 is faster up to 1536 rows (128, 164) but puts up to three times
+//    the rounding on the nearly singular lines (16 x 96 x 1536, all periodic:
+//    1.5e-11, 5.4e-12), so it is left to the tuner;
 //  * longer lines one thread a line (k_zthomas, where the reason stands).
 template <typename T>
 int z_default(int n3m, int nwg16) {
     if (n3m > 2048) return 6;
-    if (n3m > 1024) return n3m <= 1536 ? 14 : 4;
+    if (n3m > 1024) return 4;
     if (nwg16 < 4 * num_cus()) return n3m <= 400 ? 5 : (n3m <= 512 ? 2 : (n3m <= 768 ? 13 : 4));
     if (n3m <= 24) return 11;
     if (sizeof(T) == 4 && n3m <= 256) return n3m <= 128 ? 16 : 15;
