@@ -28,6 +28,7 @@ struct GateTest {
     double tol = 0.0;
     int count = 0;
     double *res_out = nullptr;
+    bool nan_closes = false;  // a NaN residual closes the gate (the host sees it)
 };
 static __global__ void __launch_bounds__(256) k_reduce3(const double *__restrict__ partial, int n, double *__restrict__ out,
                                                  const int *__restrict__ gate, GateTest check = GateTest{},
@@ -56,7 +57,7 @@ static __global__ void __launch_bounds__(256) k_reduce3(const double *__restrict
             const double rel = b > 0 ? sqrt(a / b) : sqrt(a);
             *check.res_out = rel;
             check.gate[1] += check.count;
-            check.gate[0] = (rel <= check.tol) ? 0 : 1;
+            check.gate[0] = (rel <= check.tol || (check.nan_closes && rel != rel)) ? 0 : 1;
         }
     }
 }

@@ -96,9 +96,9 @@ struct ppf_plan {
     double *partial = nullptr;  // residual partial sums
     double *red = nullptr;      // residual totals: sum r^2, sum f^2, sum p (3)
     int npartial = 0;
-    double *hred = nullptr;     // pinned host copy of red (refinement convergence test)
-    int *dgate = nullptr;       // device refinement test: [0] more sweeps needed, [1] sweeps run
-    double *dres = nullptr;     // device refinement test: last relative residual
+    double *hred = nullptr;     // pinned host copies of red (refinement convergence tests)
+    int *dgate = nullptr;       // device refinement test: [0] more sweeps needed, [1] sweeps run; [2], [3] the same of the host-tested solve's first sweep
+    double *dres = nullptr;     // device refinement test: last relative residual, [1] as above
     const int *gate = nullptr;  // gate the launch helpers pass (nullptr: kernels always run)
     ppf::AxisTables<double> tx64, ty64;
     ppf::AxisTables<float> tx32, ty32;

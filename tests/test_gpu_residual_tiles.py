@@ -74,3 +74,40 @@ def test_refined_ghost_layers(n, pbc, pz):
                     s = (p + q) ** 2
                     v[g] = s / (s - p * p) * v[i] - p * p / (s - p * p) * v[j]
     assert np.abs(got - want).max() <= 1e-14 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("n", [(16, 12, 10), (96, 64, 40)])
+def test_first_correction_launched_ahead_of_its_test(n):
+    """Below a tol of 1e-9 the first correction is launched with its test, gated
+    by it: the bits and the sweep count of the solve that waits for the test
+    (a tol just above), none for a zero or a NaN right-hand side, and further
+    sweeps, or a miss, where one is not enough."""
+    axes = _axes(n, (False, True, False))
+    f = np.random.default_rng(sum(n)).standard_normal(n[::-1])
+    w = axes[2].dx[1:n[2] + 1]
+    f -= float(np.einsum("kji,k->", f, w)) / (w.sum() * n[0] * n[1])
+
+    def run(rhs, tol, sweeps=8):
+        plan = api.FFTPoisson(*n, tuple(a.L for a in axes), (False, True, False), precision=api.PPF_PREC_FP32_IR,
+                              tol=tol, max_sweeps=sweeps)
+        dev = api.Problem3D(rhs, *axes)
+        try:
+            st = plan.solve(dev.rhs, dev.p, dev.dmx1, dev.dmx2, dev.dmx3, dev.dx3, allow_not_converged=True)
+            api.sync()
+            return dev.p.download(), st.sweeps, st.rel_residual
+        finally:
+            dev.free()
+            plan.clean()
+
+    waits, ahead = run(f, 1.01e-9), run(f, 0.99e-9)
+    assert ahead[1] == waits[1] == 1 and ahead[2] == waits[2] <= 0.99e-9
+    np.testing.assert_array_equal(ahead[0], waits[0])
+    assert run(f, 1e-30, 1)[1:] == waits[1:]  # the cap ends it after one, above tol
+    more = run(f, 1e-30, 3)
+    assert more[1] == 3 and more[2] <= waits[2]
+    zero = run(np.zeros_like(f), 1e-10)
+    assert zero[1:] == (0, 0.0) and not zero[0].any()
+    g = f.copy()
+    g[0, 0, 0] = np.nan
+    bad = run(g, 1e-10)
+    assert bad[1] == 0 and np.isnan(bad[2])
