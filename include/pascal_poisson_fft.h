@@ -147,8 +147,10 @@ int ppf_solve_async_result(ppf_plan *plan, void *stream, ppf_stats *stats);
  * extents, the x- and y-pass variants (threads per line: one radix-R
  * butterfly per thread per stage, or half the threads with two) and the
  * z-pass kernel shapes (partitioned Thomas with K rows per thread and S
- * columns per workgroup); keeps the fastest of each pass for later solves and returns the z shape's id in
- * *zvariant (may be NULL).  Results are cached per problem shape (extents,
+ * columns per workgroup; FP64 lines over 1024 rows without the shape that is
+ * fastest there but less accurate, and over 2048 rows one thread per line);
+ * keeps the fastest of each pass for later solves and returns the z shape's
+ * id in *zvariant (may be NULL).  Results are cached per problem shape (extents,
  * boundary conditions, precision) for the life of the process: a second plan
  * of a tuned shape is set without timing.  p is overwritten.  Synchronises
  * the stream.  Replaces the reference's fixed thread shapes threads_tdma /

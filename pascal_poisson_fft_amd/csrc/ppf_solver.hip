@@ -496,11 +496,21 @@ int ppf_plan_tune(ppf_plan *p, const double *prhs, double *P, const double *dmx1
     p->xvariant = vxf;
     p->xvinv = vxi;
     p->yvariant = vy;
-    // z pass: the (K,S) shapes (9 and 10 are 4 and 3 again)
-    static const int cand[] = {3, 1, 2, 4, 5, 7, 8, 11, 12, 13, 14, 15, 16, 17};
+    // z pass: the (K,S) shapes (9 and 10 are 4 and 3 again) and, above 2048
+    // rows, the one-thread-per-line kernel, whose scratch such plans hold.
+    // Not by time alone: on FP64 lines over 1024 rows K = 48 (14) is the
+    // fastest shape (16 x 96 lines of 1536 rows 27 us, K = 24 35, K = 32 38;
+    // of 2050 rows 53, one thread a line 265) but its longer sweeps put more
+    // rounding on the nearly singular lines: relative error of those solves,
+    // uniform and periodic, against an 80-bit z solve, 2.0e-11, 1.4e-11 and
+    // 7.5e-12 at 1536 rows, 3.9e-11 and 1.9e-12 at 2050.
+    static const int cand[] = {3, 1, 2, 4, 5, 6, 7, 8, 11, 12, 13, 14, 15, 16, 17};
+    const int n3m = p->d.n3m;
     int best = 0;
     float best_ms = 0.f;
     for (int v : cand) {
+        if (v == 6 && n3m <= 2048) continue;
+        if (v == 14 && n3m > 1024 && p->d.precision == PPF_PREC_FP64) continue;
         p->zvariant = v;
         float st[5];
         const int rc = time_stages(st);

@@ -208,3 +208,38 @@ def test_tuner_caches_per_shape_and_keeps_parity():
         for pl in plans:
             pl.clean()
         dev.free()
+
+
+@pytest.mark.parametrize("n3", [1026, 1400, 1536, 2050, 2544])
+def test_tuned_long_lines_keep_their_accuracy(n3):
+    """FP64 lines over 1024 rows: the tuner does not trade accuracy for time.
+    K = 48 is the fastest shape there, and on these (uniform, periodic x and y)
+    up to 2e-11 away from an 80-bit z solve at 1536 rows and 4e-11 at 2050,
+    where K = 24 and 32 and one thread per line stay within the 1e-11 of lines
+    this long.  Over 2048 rows the tuned plan runs what an untuned one does."""
+    n1, n2, L = 16, 96, (2.0, 2.0, 2.0)
+    ax, ay, az = make_axis(n1, L[0], True), make_axis(n2, L[1], True), make_axis(n3, L[2], False)
+    f = np.random.default_rng(0).standard_normal((n3, n2, n1))
+    f -= f.mean()
+    plan = api.FFTPoisson(n1, n2, n3, L, (True, True, False))
+    dev = api.Problem3D(f, ax, ay, az)
+    args = (dev.rhs, dev.p, dev.dmx1, dev.dmx2, dev.dmx3, dev.dx3)
+    try:
+        plan.solve(*args)
+        api.sync()
+        default = dev.p.download()
+        v = plan.tune(*args)
+        print(f"n3m={n3} tuned z shape {v}", flush=True)
+        dev.p.fill_zero()
+        plan.solve(*args)
+        api.sync()
+        got = dev.p.download()
+    finally:
+        dev.free()
+        plan.clean()
+    if n3 > 2048:
+        assert v == 6 and np.array_equal(got, default)
+        return
+    assert v in (4, 13)
+    ref = O.solve(f, L, (True, True, False), ax.dmx, ay.dmx, az.dmx, az.dx)
+    assert float(np.linalg.norm(got - ref) / np.linalg.norm(ref)) <= 1e-11
