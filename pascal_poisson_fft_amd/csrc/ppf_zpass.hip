@@ -22,25 +22,43 @@ namespace {
 //    128-byte rows: 256 rows (32,32) 44, (16,16) 58; 128 rows (16,32) 22,
 //    (8,16) 28; 512 rows (32,32) 109, (32,16) 135 (512^3: 345, 405); 384 rows
 //    (32,32) 90, (24,16) 81;
-//  * fewer workgroups than four per CU (they are all resident at once, so a
-//    line's chain of rows is what counts): 8 columns and short partitions.
-//    64 x 64 lines (PP) of 64 rows: (8,8) 7.7, (16,16) 8.5, (32,16) 10.5; of
-//    512 rows (16,8) 14.7, (8,8) 17.0, (32,16) 15.9; of 768 rows (24,8) 20,
-//    (24,16) 21, (32,16) 29; of 1024 rows (32,8) 28, (32,16) 34;
+//  * fewer workgroups than four per CU are all resident at once, so a line's
+//    chain of rows is what counts: 8 columns and short partitions, but only as
+//    long as twice as many workgroups are resident too, which ends the earlier
+//    the longer the line (and for FP32, whose 8 columns are a quarter of a
+//    128-byte row); the lines below lie there.  32 x 32, 64 x 64, 64 x 80 and
+//    120 x 120 lines (64, 256, 320, 960 workgroups):
+//      66 rows (8,8) 7.4 8.6 - 12.4, (16,16) 8.7 9.1 - 13.2;
+//      256 rows (8,8) 8.3 10.4 10.6 22.7, (16,16) 9.4 11.1 11.4 16.4;
+//      300 rows (8,8) 9.5 11.6 13.1 27.8, (20,16) 9.9 11.8 12.2 19.7;
+//      512 rows (16,8) 10.2 13.8 15.4 42.0, (32,16) 12.6 15.2 16.0 30.2;
+//      768 rows (24,8) 12.4 16.9 24.0 63.7, (24,16) 15.2 18.0 20.8 42.6;
+//      1024 rows (32,8) 14.8 20.1 31.0 84.1, (32,16) 18.0 21.4 34.1 72.7;
+//      FP32 of 768 rows (24,8) 11.6 18.3 21.3 75.1, (24,16) 13.6 15.1 19.2 36.0;
+//      of 1024 rows (32,8) 13.6 25.8 33.7 105, (32,16) 15.7 18.1 29.2 65;
 //  * 1025..2048 rows 8 columns (a 16-column workgroup exceeds 512 threads or
 //    its registers) and K = 32: 128 x 128 lines of 2048 rows 201, K=48 220.
 //    K = 48 is faster up to 1536 rows (128, 164) but puts up to three times
 //    the rounding on the nearly singular lines (16 x 96 x 1536, all periodic:
-//    1.5e-11, 5.4e-12), so it is left to the tuner;
+//    1.5e-11, 5.4e-12), so neither this rule nor, for FP64, the tuner takes it;
 //  * longer lines one thread a line (k_zthomas, where the reason stands).
 template <typename T>
 int z_default(int n3m, int nwg16) {
     if (n3m > 2048) return 6;
     if (n3m > 1024) return 4;
-    if (nwg16 < 4 * num_cus()) return n3m <= 400 ? 5 : (n3m <= 512 ? 2 : (n3m <= 768 ? 13 : 4));
-    if (n3m <= 24) return 11;
-    if (sizeof(T) == 4 && n3m <= 256) return n3m <= 128 ? 16 : 15;
-    if (sizeof(T) == 4 && n3m > 416 && n3m <= 512) return 15;
+    constexpr bool F32 = sizeof(T) == 4;
+    const int cus = num_cus();
+    if (nwg16 < 4 * cus) {
+        const bool few = 2 * nwg16 <= 3 * cus, fewer = nwg16 <= (F32 ? cus / 2 : cus);
+        if (n3m <= 256) return nwg16 <= (n3m <= 128 ? 4 : n3m <= 192 ? 3 : 2) * cus ? 5 : 1;
+        if (n3m <= 320) return fewer ? 5 : 7;
+        if (n3m <= 512 && few) return 2;
+        if (n3m > 512 && (F32 ? fewer : few)) return n3m <= 768 ? 13 : 4;
+    } else {
+        if (n3m <= 24) return 11;
+        if (F32 && n3m <= 256) return n3m <= 128 ? 16 : 15;
+        if (F32 && n3m > 416 && n3m <= 512) return 15;
+    }
     if (n3m <= 64) return 1;
     if (n3m <= 128) return 11;
     if (n3m <= 320) return 7;

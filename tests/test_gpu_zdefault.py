@@ -63,3 +63,33 @@ def test_one_thread_per_line_matches_oracle(n3, precision):
     err = _solve(20, 12, n3, (n3 % 4 == 2, n3 % 8 >= 4), precision, zvariant=6)
     bar = 1e-12 if precision == api.PPF_PREC_FP64 else 5e-6
     assert err <= bar, err
+
+
+@pytest.mark.parametrize("precision", [api.PPF_PREC_FP64, api.PPF_PREC_FP32_IR], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("n3", [192, 194, 256, 258, 320, 322, 384, 386, 448, 450, 512, 514, 768, 770, 1024])
+def test_default_z_shape_of_middle_grids(n3, precision):
+    """Between one and four 16-column workgroups per CU (120 x 96: 768 with
+    walls in x and y, on 256 CUs) lines over 192 rows take 16 columns a
+    workgroup, the same bits as the shape pinned: 8 columns made them up to a
+    third slower there."""
+    n1, n2, L = 120, 96, (2.0, 3.0, 1.5)
+    ax, ay, az = make_axis(n1, L[0], False), make_axis(n2, L[1], False), make_axis(n3, L[2], False)
+    f = np.random.default_rng(n3).standard_normal((n3, n2, n1))
+    plan = api.FFTPoisson(n1, n2, n3, L, (False, False, False), precision=precision)
+    dev = api.Problem3D(f - f.mean(), ax, ay, az)
+    shape = next(v for rows, v in ((192, 5), (256, 1), (320, 7), (384, 12), (448, 17), (512, 3), (768, 12), (1024, 3))
+                 if n3 <= rows)
+    got = []
+    try:
+        for v in (0, shape):
+            plan.set_zvariant(v)
+            plan.solve_sweeps(dev.rhs, dev.p, dev.dmx1, dev.dmx2, dev.dmx3, dev.dx3, 0)
+            api.sync()
+            got.append(dev.p.download())
+    finally:
+        dev.free()
+        plan.clean()
+    ref = O.solve(f - f.mean(), L, (False, False, False), ax.dmx, ay.dmx, az.dmx, az.dx)
+    err = float(np.linalg.norm(got[0] - ref) / np.linalg.norm(ref))
+    bar = (1e-12 if n3 <= 512 else 1e-11) if precision == api.PPF_PREC_FP64 else 5e-6
+    assert np.array_equal(got[0], got[1]) and err <= bar, err
