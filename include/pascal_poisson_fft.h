@@ -160,8 +160,10 @@ int ppf_plan_tune(ppf_plan *plan, const double *prhs, double *p, const double *d
                   const double *dmx3, const double *dx3, void *stream, int *zvariant);
 
 /* Pins the z-pass kernel shape (an id returned by ppf_plan_tune, 1..17; 0 =
- * the default chosen by the extents).  A shape that does not fit the plan's z extent
- * makes later solves return PPF_ERR_UNSUPPORTED. */
+ * the default chosen by the extents).  A shape that does not fit the plan's z
+ * extent makes later solves return PPF_ERR_UNSUPPORTED; with periodic z, 7..11
+ * and 17 stand for shape 3 (4 over 1024 rows) past 512, 512, 1024, 1024, 256
+ * and 768 rows. */
 int ppf_plan_set_zvariant(ppf_plan *plan, int zvariant);
 
 /* The plan's pass variants: variants[0] x passes, [1] y pass (0/1 as for

@@ -202,6 +202,13 @@ inline EigGeom eig_geom(const ppf_plan *p) {
 // z-pass shapes: 6 one thread per line (k_zthomas), the others (K, S) shapes
 // of k_zpart; 0 = chosen by the extents (z_default).
 constexpr int kZVariants = 17;
+// Rows up to which ids 7..11 and 17 mean their own shape (the others are bound
+// by threads and LDS alone).  These are the extents the ids have always taken;
+// past them a pin is refused with walls in z, and with periodic z, where it was
+// always accepted, stands for shape 3 or 4.
+constexpr int z_rows(int v) {
+    return v == 7 || v == 8 ? 512 : v == 9 || v == 10 ? 1024 : v == 11 ? 256 : v == 17 ? 768 : 4096;
+}
 // x-pass variants (XGeom): 0 and 1 threads per line, 2 without the register
 // prefetch, 3 the same kernel as 2 with one workgroup per tile (not
 // persistent); y-pass variants (YGeom): 0 and 1.

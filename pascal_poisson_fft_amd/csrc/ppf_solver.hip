@@ -509,7 +509,7 @@ int ppf_plan_tune(ppf_plan *p, const double *prhs, double *P, const double *dmx1
     int best = 0;
     float best_ms = 0.f;
     for (int v : cand) {
-        if (v == 6 && n3m <= 2048) continue;
+        if (n3m > z_rows(v) || (v == 6 && n3m <= 2048)) continue;
         if (v == 14 && n3m > 1024 && p->d.precision == PPF_PREC_FP64) continue;
         p->zvariant = v;
         float st[5];

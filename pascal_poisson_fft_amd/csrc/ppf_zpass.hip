@@ -90,15 +90,15 @@ int launch_z(ppf_plan *p, T *W, const double *dx3, const double *dmx3, hipStream
     z.gate = p->gate;
     const int n3m = p->d.n3m;
     // partitioned register-resident Thomas, shape (K rows per thread, S
-    // columns per workgroup); launched only when S*P <= NTMAX, the LDS
-    // footprint stays within 64 KB and n3m within `most`
+    // columns per workgroup); launched only when S*P <= NTMAX and the LDS
+    // footprint stays within 64 KB
     bool done = false;
-    auto part = [&](auto kk, auto ss, auto nt, auto wpe, int most = 4096) {
+    auto part = [&](auto kk, auto ss, auto nt, auto wpe) {
         constexpr int K = decltype(kk)::value, S = decltype(ss)::value;
         constexpr int NTMAX = decltype(nt)::value, WPE = decltype(wpe)::value;
         const int P = (n3m + K - 1) / K;
         const size_t shm = zp_lds_bytes<K, S>(P);
-        if (P < 1 || S * P > NTMAX || shm > 65536 || n3m > most) return;
+        if (P < 1 || S * P > NTMAX || shm > 65536) return;
         const int tiles = (p->Lx + S - 1) / S;
         const int ntiles = tiles * p->znjr;
         // FP64 arithmetic for FP32 storage too: FP32 arithmetic measured no
@@ -110,17 +110,18 @@ int launch_z(ppf_plan *p, T *W, const double *dx3, const double *dmx3, hipStream
     using std::integral_constant;
 #define PPF_Z(K, S, NT, WPE) integral_constant<int, K>{}, integral_constant<int, S>{}, integral_constant<int, NT>{}, integral_constant<int, WPE>{}
     int v = p->zvariant ? p->zvariant : z_default<T>(n3m, (p->Lx + 15) / 16 * p->znjr);
-    // with periodic z a pin of the shapes below whose extent is limited means
-    // the shape without that limit
-    if (z.zper && ((v >= 7 && v <= 11) || v == 17) && p->zvariant) v = n3m <= 1024 ? 3 : 4;
+    if (n3m > z_rows(v)) {
+        if (!z.zper) return PPF_ERR_UNSUPPORTED;
+        v = n3m <= 1024 ? 3 : 4;
+    }
     switch (v) {
         case 1: part(PPF_Z(16, 16, 512, 4)); break;
         case 2: part(PPF_Z(16, 8, 512, 4)); break;
         case 3: case 10: part(PPF_Z(32, 16, 512, 3)); break;
-        case 4: case 9: part(PPF_Z(32, 8, 512, 3), v == 9 ? 1024 : 4096); break;
+        case 4: case 9: part(PPF_Z(32, 8, 512, 3)); break;
         case 5: part(PPF_Z(8, 8, 512, 4)); break;
-        case 7: part(PPF_Z(20, 16, 512, 4), 512); break;
-        case 8: part(PPF_Z(12, 16, 704, 4), 512); break;
+        case 7: part(PPF_Z(20, 16, 512, 4)); break;
+        case 8: part(PPF_Z(12, 16, 704, 4)); break;
         case 11: part(PPF_Z(8, 16, 512, 4)); break;
         case 12: part(PPF_Z(24, 16, 512, 4)); break;
         case 13: part(PPF_Z(24, 8, 512, 3)); break;
@@ -128,11 +129,11 @@ int launch_z(ppf_plan *p, T *W, const double *dx3, const double *dmx3, hipStream
         // 32 columns: 128-byte row segments for FP32 workspaces
         case 15: part(PPF_Z(32, 32, 512, 3)); break;
         case 16: part(PPF_Z(16, 32, 512, 4)); break;
-        case 17: part(PPF_Z(28, 16, 512, 3), 768); break;
+        case 17: part(PPF_Z(28, 16, 512, 3)); break;
         default: break;
     }
 #undef PPF_Z
-    // a pinned shape that does not fit the extent is reported, never replaced
+    // a shape that does not fit the extent is reported
     if (!done && v != 6) return PPF_ERR_UNSUPPORTED;
     if (!done) {
         const long ncol = (long)p->Lx * p->znjr;

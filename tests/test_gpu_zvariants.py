@@ -243,3 +243,44 @@ def test_tuned_long_lines_keep_their_accuracy(n3):
     assert v in (4, 13)
     ref = O.solve(f, L, (True, True, False), ax.dmx, ay.dmx, az.dmx, az.dx)
     assert float(np.linalg.norm(got - ref) / np.linalg.norm(ref)) <= 1e-11
+
+
+def _periodic_z(n1, n2, n3, pbc, precision=api.PPF_PREC_FP64):
+    L = (2.0, 3.0, 1.5)
+    ax, ay, az = make_axis(n1, L[0], pbc[0]), make_axis(n2, L[1], pbc[1]), make_axis(n3, L[2], True)
+    f = np.random.default_rng(n1 + n3).standard_normal((n3, n2, n1))
+    f -= f.mean()
+    ref = O.solve(f, L, (pbc[0], pbc[1], True), ax.dmx, ay.dmx, az.dmx, az.dx)
+    return api.FFTPoisson(n1, n2, n3, L, (pbc[0], pbc[1], True), precision=precision), api.Problem3D(f, ax, ay, az), ref
+
+
+def _pinned(plan, dev, v):
+    plan.set_zvariant(v)
+    dev.p.fill_zero()
+    plan.solve_sweeps(dev.rhs, dev.p, dev.dmx1, dev.dmx2, dev.dmx3, dev.dx3, 0)
+    api.sync()
+    return dev.p.download()
+
+
+def test_periodic_z_runs_the_pinned_shape():
+    """With periodic z an id means its own shape up to its rows, as with walls:
+    the bits of the default where the default is that shape (20 rows by 16
+    columns at 200 rows of a large grid), not those of shape 3.  Past its rows
+    it stands for shape 3, or 4 over 1024 rows."""
+    plan, dev, ref = _periodic_z(160, 120, 200, (True, False))
+    try:
+        default, k20, k32 = (_pinned(plan, dev, v) for v in (0, 7, 3))
+    finally:
+        dev.free()
+        plan.clean()
+    assert np.linalg.norm(default - ref) <= 1e-12 * np.linalg.norm(ref)
+    assert np.array_equal(k20, default) and not np.array_equal(k20, k32)
+    for n3, ids, same in ((600, (7, 8, 11), 3), (1030, (7, 9, 10, 17), 4)):
+        plan, dev, _ = _periodic_z(16, 12, n3, (False, False))
+        try:
+            want = _pinned(plan, dev, same)
+            for v in ids:
+                assert np.array_equal(_pinned(plan, dev, v), want), (n3, v)
+        finally:
+            dev.free()
+            plan.clean()
