@@ -1,6 +1,7 @@
 """Residual tiles (64 cells of a wave, TY rows, kz planes) and the ghost layers
 re-derived after refinement, at extents where a wave, a row block or a plane
-block is cut short.
+block is cut short; on 256 CUs the last three take blocks of 4 rows by 8 planes,
+2 by 8 and 8 by 16, the smaller ones 2 by 4.
 
 The residual is a sum of squares of FP64 differences: against the oracle's, on a
 random iterate, 1e-12 relative (as in the other residual tests).  The ghost
@@ -26,7 +27,8 @@ def _axes(n, pbc):
 
 @pytest.mark.parametrize("pbc", BCS, ids=["NN", "PP", "PN", "NP"])
 @pytest.mark.parametrize("n", [(8, 8, 2), (10, 10, 6), (64, 10, 34), (80, 24, 18), (128, 12, 66), (320, 14, 10),
-                               (192, 192, 40), (480, 240, 98)])
+                               (192, 192, 40), (480, 240, 98), (480, 30, 300),
+                               (480, 240, 290)])
 def test_residual_tiles_match_oracle(n, pbc):
     ax, ay, az = _axes(n, pbc + (False,))
     rng = np.random.default_rng(sum(n))

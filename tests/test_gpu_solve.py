@@ -91,10 +91,9 @@ def test_c1_manufactured_64():
 @pytest.mark.parametrize("pbc", BCS, ids=["NN", "PP", "PN", "NP"])
 @pytest.mark.parametrize("n1,n2,n3", [(32, 24, 16), (96, 20, 40), (320, 10, 34), (160, 28, 6), (64, 12, 70)])
 def test_gpu_residual_matches_oracle(pbc, n1, n2, n3):
-    """The residual kernel on a random iterate: y blocks of 8, 4 and 2 rows
-    (n2m = 24; 20, 12, 28; 10 -- extents are even, so never 1), one and two x
-    tiles with the last cell inside a wave (n1m = 32, 160), z blocks shorter
-    than 32 planes, every x/y branch.
+    """The residual kernel on a random iterate at small extents, which take
+    blocks of 2 rows by 4 planes: one to five x tiles of 64 cells with the last
+    one whole or cut (n1m = 32, 96, 160), a cut last z block, every x/y branch.
     A wrong neighbour in any row or column of cells moves the sum of r^2 by
     far more than the 1e-12 bound."""
     ax, ay, az, f = _problem(n1, n2, n3, pbc, False, 1.2, 3)
@@ -111,9 +110,8 @@ def test_gpu_residual_matches_oracle(pbc, n1, n2, n3):
 @pytest.mark.parametrize("pbc", [(False, False), (True, True)], ids=["NN", "PP"])
 @pytest.mark.parametrize("n1,n2,n3", [(512, 256, 512), (512, 256, 256), (512, 256, 128)])
 def test_gpu_residual_row_blocks_match_oracle(pbc, n1, n2, n3):
-    """Shapes large enough that the residual kernel blocks 8, 4 and 2 rows per
-    thread (it keeps at least 4 tiles per CU on a 256-CU device: 512 x 256 x
-    512, 256, 128 cells give 8, 4, 2)."""
+    """Shapes large enough that every CU has 16 waves of tiles (on 256 CUs):
+    blocks of 8 rows by 32 planes, 8 by 16 and 4 by 16."""
     ax, ay, az, f = _problem(n1, n2, n3, pbc, False, 1.2, 5)
     P = np.random.default_rng(6).standard_normal((n3 + 2, n2 + 2, n1 + 2))
     plan = api.FFTPoisson(n1, n2, n3, (ax.L, ay.L, az.L), (pbc[0], pbc[1], False))

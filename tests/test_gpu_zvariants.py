@@ -1,18 +1,18 @@
 """Every z-pass kernel shape, pinned with ppf_plan_set_zvariant, against the
 FP64 oracle.
 
-The autotuner may return any of these shapes, so each one must be correct on
-its own, at z extents that stress its partitioning: 96 (the tuner test's
-extent), 136 and 144 (partial last wavefront for the pipelined K=16 forms),
-270 (partial wavefront for K=32 pipelined forms, ragged last partition), 768
-(the projection stream's extent), 1500 (above 1024, where the default is the
-K=32, S=8 shape) -- and 2050, where only the one-thread-per-line Thomas
-runs.  Both z-row layouts are covered: Neumann y (rows 1..n2m) and periodic y
-with Neumann x (R2C columns, rows 0..n2m+1).
+The autotuner may return these shapes, so each one must be correct on its own,
+at z extents that stress its partitions (K rows a thread: 8, 12, 16, 20, 24, 28,
+32, 48): 96, 240, 504 and 512 (whole last partitions of one K or another), 136,
+144, 168 and 270 (a cut last partition, down to 2 rows), 768 (the projection
+stream's extent), 1500 (above 1024, where the default is K = 32 and 8 columns)
+-- and 2050, where an FP64 plan runs the one-thread-per-line Thomas.  Both z-row
+layouts are covered: Neumann y (rows 1..n2m) and periodic y with Neumann x (R2C
+columns, rows 0..n2m+1).
 
-A shape that does not fit an extent (its partitions exceed the workgroup or
-its reduced system the wavefront) is rejected with PPF_ERR_UNSUPPORTED, never
-run; the test records which.
+A shape that does not fit an extent (its partitions exceed the workgroup or its
+rows the id's) is rejected with PPF_ERR_UNSUPPORTED, never run; the test records
+which.
 
 Tolerance: <= 1e-12 relative L2 of the ghosted solution against the oracle
 for z lines of up to 1024 rows.  Longer stretched lines are worse conditioned
@@ -23,10 +23,7 @@ that much; there the bar is 1e-11.  As a check against gross errors (a wrong
 row or sign leaves a residual of order one) every solve must also leave an
 FP64 relative residual <= max(1e-11, twice the oracle's own): on long
 stretched lines the oracle's residual itself is about 2e-12, because the
-operator's coefficients span several orders of magnitude.  (Measured at 768
-rows: the partitioned shapes leave <= 0.5e-12, the pipelined K=32 shapes
-2-3.5e-12, their 2P-row reduced system being solved without the halving and
-unit-diagonal scaling of the partitioned form.)
+operator's coefficients span several orders of magnitude.
 """
 import numpy as np
 import pytest
@@ -61,7 +58,7 @@ def _case(n1, n2, n3, pbc, seed):
 
 
 @pytest.mark.parametrize("pbc", [(False, False), (False, True)], ids=["NN", "NP"])
-@pytest.mark.parametrize("n3", [96, 136, 144, 270, 768, 1500])
+@pytest.mark.parametrize("n3", [96, 136, 144, 168, 240, 270, 504, 512, 768, 1500])
 def test_every_zvariant_matches_oracle(pbc, n3):
     n1, n2 = 24, 16
     L, ax, ay, az, f, ref = _case(n1, n2, n3, pbc, seed=n3 + 7 * pbc[1])
@@ -284,3 +281,59 @@ def test_periodic_z_runs_the_pinned_shape():
         finally:
             dev.free()
             plan.clean()
+
+
+@pytest.mark.parametrize("n3", [30, 270, 512, 1500, 2544])
+def test_every_zvariant_fp32(n3):
+    """The same shapes on FP32 workspaces (one solve without corrections), up
+    to the last rows K = 48 takes: storage rounding of 6e-8 a pass over five
+    passes, bounded by 5e-6 as a gross-error bar."""
+    n1, n2, pbc = 24, 16, (True, False)
+    L, ax, ay, az, f, ref = _case(n1, n2, n3, pbc, seed=n3)
+    plan = api.FFTPoisson(n1, n2, n3, L, (True, False, False), precision=api.PPF_PREC_FP32_IR)
+    dev = api.Problem3D(f, ax, ay, az)
+    ran = []
+    try:
+        for v in VARIANTS:
+            try:
+                got = _pinned(plan, dev, v)
+            except api.PPFError as e:
+                assert e.code == UNSUPPORTED, e
+                continue
+            err = float(np.linalg.norm(got - ref) / np.linalg.norm(ref))
+            assert err <= 5e-6, (v, err)
+            ran.append(v)
+    finally:
+        dev.free()
+        plan.clean()
+    assert {6, 14} <= set(ran)
+
+
+@pytest.mark.parametrize("pbc", [(False, False), (True, True), (True, False), (False, True)],
+                         ids=["NN", "PP", "PN", "NP"])
+@pytest.mark.parametrize("n3", [8, 30, 96, 200, 256, 270, 512, 768, 1022])
+def test_every_zvariant_periodic_z(pbc, n3):
+    """Every shape that takes these rows with periodic z: whole last partitions
+    and cut ones for each K, the wrapped end planes of z among the compared
+    values (an FP64 solve writes them in the z pass).  1e-12 up to 270 rows and
+    1e-11 above: on these uniform lines the oracle's FP64 cyclic Thomas is off
+    an 80-bit z solve by 1.2e-12 at 256 rows already, 4.3e-12 at 512 and
+    1.3e-11 at 768."""
+    plan, dev, ref = _periodic_z(24, 16, n3, pbc)
+    ran = []
+    try:
+        for v in VARIANTS:
+            try:
+                got = _pinned(plan, dev, v)
+            except api.PPFError as e:
+                assert e.code == UNSUPPORTED, e
+                continue
+            err = float(np.linalg.norm(got - ref) / np.linalg.norm(ref))
+            ends = np.abs(got[[0, -1]] - got[[-2, 1]]).max() / np.abs(ref).max()
+            print(f"n3m={n3} pbc={pbc} zvariant={v} {err:.1e} {ends:.1e}", flush=True)
+            assert err <= (1e-12 if n3 <= 270 else 1e-11) and ends <= 1e-13, (v, err, ends)
+            ran.append(v)
+    finally:
+        dev.free()
+        plan.clean()
+    assert {3, 6, 9, 10} <= set(ran)
