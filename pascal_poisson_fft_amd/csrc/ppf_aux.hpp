@@ -102,7 +102,7 @@ static __global__ void __launch_bounds__(256) k_ghosts(double *__restrict__ P, G
         ws[threadIdx.x][1] = d1 * d1 / (s * s - d1 * d1);
     }
     __syncthreads();
-    unsigned q = blockIdx.x * blockDim.x + threadIdx.x;  // (extents up to 1024, 1024 and 4096: 2^24 cells in all)
+    unsigned q = blockIdx.x * blockDim.x + threadIdx.x;  // (extents up to 1024, 1024 and 4096: below 2^25 cells in all)
     int at[3];
     if (q < 2 * nz) {
         at[2] = q < nz ? 0 : g.n[2] + 1;

@@ -1034,12 +1034,14 @@ __device__ __forceinline__ double frcp(double x) {
 //    waited for where it is used;
 //  * one-wave workgroups spread few lines over as many CUs.
 // z stage, 256-thread workgroups with each row's loads where they are used ->
-// this form, the same bits: 96 x 80 lines of 2050 rows 1589 -> 277 us, 128 x
-// 128 1804 -> 355, 256 x 256 of 2052 2533 -> 1356, 64 x 64 of 512 401 -> 73.
-// One row of 64 lines an operation: 302, 335, 1270, 81; four of 16: 291, 456,
-// 1362, 77.  (The partitioned form of k_zpart takes 130 us on the first of
-// these, but adds up to 1.6e-11 to lines this long, which is more than FP64
-// solves are held to.)
+// this form: 96 x 80 lines of 2050 rows 1589 -> 277 us, 128 x 128 1804 -> 355,
+// 256 x 256 of 2052 2533 -> 1356, 64 x 64 of 512 401 -> 73.  The same operations
+// but for the pivot's reciprocal, frcp for an IEEE division, which may differ in
+// its last bit (those solutions did not).  One row of 64 lines an operation:
+// 302, 335, 1270, 81; four of 16: 291, 456, 1362, 77.  (The partitioned form of
+// k_zpart takes 130 us on the first of these, but is up to 3.9e-11 off an
+// 80-bit z solve on lines this long, where this one is 1.9e-12 off: 16 x 96 x
+// 2050, uniform, periodic x and y.)
 constexpr int kZtRows = 32;
 
 __device__ __forceinline__ double lane_read(double v, int lane) {

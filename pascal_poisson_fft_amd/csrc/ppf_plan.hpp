@@ -206,7 +206,7 @@ constexpr int kZVariants = 17;
 // by threads and LDS alone).  These are the extents the ids have always taken;
 // past them a pin is refused with walls in z, and with periodic z, where it was
 // always accepted, stands for shape 3 or 4.
-constexpr int z_rows(int v) {
+constexpr int z_id_rows(int v) {
     return v == 7 || v == 8 ? 512 : v == 9 || v == 10 ? 1024 : v == 11 ? 256 : v == 17 ? 768 : 4096;
 }
 // x-pass variants (XGeom): 0 and 1 threads per line, 2 without the register
@@ -250,7 +250,7 @@ inline int dispatch_y(const ppf_plan *p, T *W, const AxisTables<T> &tb, bool inv
     return inverse ? dispatch_yinv<T>(p, W, tb, dmx2, s, nplanes) : dispatch_yfwd<T>(p, W, tb, s, nplanes);
 }
 template <typename T>
-int launch_z(ppf_plan *p, T *W, const double *dx3, const double *dmx3, hipStream_t s);
+int launch_z(ppf_plan *p, T *W, hipStream_t s);
 
 // The fused batch (ppf_fused.hpp / ppf_fused.hip): every FP64 problem of a
 // batch in one persistent launch over a device work queue.

@@ -70,7 +70,7 @@ static int desc_check(const ppf_desc &d) {
     if (d.n1m <= 0 || d.n2m <= 0 || d.n3m <= 0 || !(d.L1 > 0) || !(d.L2 > 0) || !(d.L3 > 0)) return PPF_ERR_INVALID_ARG;
     if (d.precision != PPF_PREC_FP64 && d.precision != PPF_PREC_FP32_IR) return PPF_ERR_INVALID_ARG;
     // every n must be even (01_Fortran/examples/global.f90:114-120)
-    // z rows live in LDS in the z pass (2 doubles per row): n3m <= 4096
+    // n3m <= 4096 is the range the interface states and the tests cover
     if (!size_supported(d.n1m) || !size_supported(d.n2m) || d.n3m < 2 || (d.n3m & 1) || d.n3m > 4096)
         return PPF_ERR_SIZE;
     return PPF_OK;
@@ -193,7 +193,7 @@ static int run_passes(ppf_plan *p, T *W, const AxisTables<T> &tx, const AxisTabl
     if (ev) PPF_HIP(hipEventRecord(ev[1], s));
     if ((rc = dispatch_y<T>(p, W, ty, false, dmx2, s))) return rc;
     if (ev) PPF_HIP(hipEventRecord(ev[2], s));
-    if ((rc = launch_z<T>(p, W, dx3, dmx3, s))) return rc;
+    if ((rc = launch_z<T>(p, W, s))) return rc;
     if (ev) PPF_HIP(hipEventRecord(ev[3], s));
     if ((rc = dispatch_y<T>(p, W, ty, true, dmx2, s))) return rc;
     if (ev) PPF_HIP(hipEventRecord(ev[4], s));
@@ -257,11 +257,10 @@ static int refresh_ghosts(const ppf_plan *p, double *P, const double *dmx1, cons
 // The correction of one refinement sweep of an FP32_IR plan: pass 1
 // transforms the residual launch_residual(out) left in W32, passes 2-4 in
 // FP32, pass 5 adds the correction to P.  Gated by p->gate.
-static int correct32(ppf_plan *p, double *P, const double *dmx1, const double *dmx2, const double *dmx3,
-                     const double *dx3, hipStream_t s) {
+static int correct32(ppf_plan *p, double *P, const double *dmx1, const double *dmx2, hipStream_t s) {
     int rc;
     if ((rc = dispatch_xfwd<float>(p, nullptr, p->W32, p->tx32, true, s)) ||
-        (rc = dispatch_y<float>(p, p->W32, p->ty32, false, dmx2, s)) || (rc = launch_z<float>(p, p->W32, dx3, dmx3, s)) ||
+        (rc = dispatch_y<float>(p, p->W32, p->ty32, false, dmx2, s)) || (rc = launch_z<float>(p, p->W32, s)) ||
         (rc = dispatch_y<float>(p, p->W32, p->ty32, true, dmx2, s)) ||
         (rc = dispatch_xinv<float>(p, p->W32, P, p->tx32, dmx1, true, s)))
         return rc;
@@ -290,7 +289,7 @@ static int solve_fp32_ir(ppf_plan *p, const double *f, double *P, const double *
     bool converged = false;
     if (tol < 0) {
         for (; sweeps < maxs; ++sweeps)
-            if ((rc = launch_residual(p, f, P, s, true)) || (rc = correct32(p, P, dmx1, dmx2, dmx3, dx3, s))) return rc;
+            if ((rc = launch_residual(p, f, P, s, true)) || (rc = correct32(p, P, dmx1, dmx2, s))) return rc;
         if (sweeps > 0 && (rc = refresh_ghosts(p, P, dmx1, dmx2, dmx3, s))) return rc;
         if (stats) {
             if ((rc = ppf_residual(p, f, P, dmx3, dx3, s, &rel))) return rc;
@@ -322,7 +321,7 @@ static int solve_fp32_ir(ppf_plan *p, const double *f, double *P, const double *
             if ((rc = launch_residual(p, f, P, s, true, true, GateTest{gate, tol, 0, p->dres + 1, true}, p->hred)))
                 return rc;
             p->gate = gate;
-            if ((rc = correct32(p, P, dmx1, dmx2, dmx3, dx3, s)) ||
+            if ((rc = correct32(p, P, dmx1, dmx2, s)) ||
                 (rc = launch_residual(p, f, P, s, false, true, GateTest{}, p->hred + 3)))
                 return rc;
         }
@@ -339,7 +338,7 @@ static int solve_fp32_ir(ppf_plan *p, const double *f, double *P, const double *
             if (rel <= tol) { converged = true; break; }
             if (sweeps == maxs || !(rel == rel)) break;
             if ((waiting || !store) && (rc = launch_residual(p, f, P, s, true, false))) return rc;
-            if ((rc = correct32(p, P, dmx1, dmx2, dmx3, dx3, s))) return rc;
+            if ((rc = correct32(p, P, dmx1, dmx2, s))) return rc;
             ++sweeps;
         }
         if (sweeps > 0 && (rc = refresh_ghosts(p, P, dmx1, dmx2, dmx3, s))) return rc;
@@ -375,7 +374,7 @@ static int solve_fp32_async(ppf_plan *p, const double *f, double *P, const doubl
     if ((rc = run_passes<float>(p, p->W32, p->tx32, p->ty32, f, P, dmx1, dmx2, dmx3, dx3, s, nullptr))) return rc;
     // the z row table of this solve (filled by pass 1) serves the residuals
     for (int i = 0; i < nmin; ++i)
-        if ((rc = launch_residual(p, f, P, s, true)) || (rc = correct32(p, P, dmx1, dmx2, dmx3, dx3, s))) return rc;
+        if ((rc = launch_residual(p, f, P, s, true)) || (rc = correct32(p, P, dmx1, dmx2, s))) return rc;
     // each test without the FP32 store of r; a gated residual with the store
     // feeds the gated correction (both return at once once the gate closed)
     for (int i = nmin;; ++i) {
@@ -383,7 +382,7 @@ static int solve_fp32_async(ppf_plan *p, const double *f, double *P, const doubl
         if ((rc = launch_residual(p, f, P, s, false, true, GateTest{p->dgate, tol, i > nmin ? 1 : 0, p->dres})))
             return rc;
         if (i >= nmax) break;
-        if ((rc = launch_residual(p, f, P, s, true, false)) || (rc = correct32(p, P, dmx1, dmx2, dmx3, dx3, s)))
+        if ((rc = launch_residual(p, f, P, s, true, false)) || (rc = correct32(p, P, dmx1, dmx2, s)))
             return rc;
     }
     p->gate = nullptr;
@@ -509,7 +508,7 @@ int ppf_plan_tune(ppf_plan *p, const double *prhs, double *P, const double *dmx1
     int best = 0;
     float best_ms = 0.f;
     for (int v : cand) {
-        if (n3m > z_rows(v) || (v == 6 && n3m <= 2048)) continue;
+        if (n3m > z_id_rows(v) || (v == 6 && n3m <= 2048)) continue;
         if (v == 14 && n3m > 1024 && p->d.precision == PPF_PREC_FP64) continue;
         p->zvariant = v;
         float st[5];

@@ -21,7 +21,9 @@ namespace {
 //  * FP32 workspaces up to 256 and near 512 rows take 32 columns, whole
 //    128-byte rows: 256 rows (32,32) 44, (16,16) 58; 128 rows (16,32) 22,
 //    (8,16) 28; 512 rows (32,32) 109, (32,16) 135 (512^3: 345, 405); 384 rows
-//    (32,32) 90, (24,16) 81;
+//    (32,32) 90, (24,16) 81.  FP64 lines never do here, though 32 columns were
+//    faster at some lengths (768 x 512 x 96 (16,32) 121, (8,16) 142; 320 x 224 x
+//    200 (32,32) 55, (20,16) 60): where was not mapped, tuned plans find it;
 //  * fewer workgroups than four per CU are all resident at once, so a line's
 //    chain of rows is what counts: 8 columns and short partitions, but only as
 //    long as twice as many workgroups are resident too, which ends the earlier
@@ -70,8 +72,8 @@ int z_default(int n3m, int nwg16) {
 }  // namespace
 
 template <typename T>
-int launch_z(ppf_plan *p, T *W, const double *dx3, const double *dmx3, hipStream_t s) {
-    // k_zpart reads the z row table that pass 1 of this solve filled
+int launch_z(ppf_plan *p, T *W, hipStream_t s) {
+    // the kernels read the z row table that pass 1 of this solve filled
     ZArgs z;
     z.Lx = p->Lx;
     z.Lxs = p->Lxs;
@@ -110,7 +112,7 @@ int launch_z(ppf_plan *p, T *W, const double *dx3, const double *dmx3, hipStream
     using std::integral_constant;
 #define PPF_Z(K, S, NT, WPE) integral_constant<int, K>{}, integral_constant<int, S>{}, integral_constant<int, NT>{}, integral_constant<int, WPE>{}
     int v = p->zvariant ? p->zvariant : z_default<T>(n3m, (p->Lx + 15) / 16 * p->znjr);
-    if (n3m > z_rows(v)) {
+    if (n3m > z_id_rows(v)) {
         if (!z.zper) return PPF_ERR_UNSUPPORTED;
         v = n3m <= 1024 ? 3 : 4;
     }
@@ -147,8 +149,7 @@ int launch_z(ppf_plan *p, T *W, const double *dx3, const double *dmx3, hipStream
     return PPF_OK;
 }
 
-
-template int launch_z<double>(ppf_plan *, double *, const double *, const double *, hipStream_t);
-template int launch_z<float>(ppf_plan *, float *, const double *, const double *, hipStream_t);
+template int launch_z<double>(ppf_plan *, double *, hipStream_t);
+template int launch_z<float>(ppf_plan *, float *, hipStream_t);
 
 }  // namespace ppf
