@@ -1,6 +1,9 @@
-"""The stand-alone Thomas at row counts around its row chunks (8 rows forward,
-16 back, one chunk ahead) and system counts around a wave: solution and overwritten c bitwise
-equal to the same operations in numpy (which rounds every one of them).
+"""The stand-alone Thomas at row counts around its row chunks (8 rows forward, 4
+in the cyclic form, 16 back; 4 and 8 up to 8 rows; one chunk ahead; loads past
+the end left out below 128 rows and clamped above) and system counts around a
+wave and around the 2^21 from which workgroups are four waves:
+solution and overwritten c bitwise equal to the same operations in numpy (which
+rounds every one of them).
 """
 import numpy as np
 import pytest
@@ -36,8 +39,9 @@ def _cyclic(a, b, c, d):
     return c, d
 
 
-@pytest.mark.parametrize("nsys", [1, 63, 130])
-@pytest.mark.parametrize("n", [1, 2, 3, 8, 9, 10, 11, 16, 17, 18, 19, 26, 32, 33, 34, 35, 50])
+@pytest.mark.parametrize("n,nsys", [(n, nsys) for n in (1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 13, 14, 16, 17, 18, 19, 26, 32, 33,
+                                                        34, 35, 50, 127, 128, 129, 136, 145) for nsys in (1, 63, 130)] +
+                         [(n, nsys) for n in (3, 6) for nsys in (2**21 - 30, 2**21 + 70)])
 def test_row_chunks_bitwise(n, nsys):
     rng = np.random.default_rng(n * 1000 + nsys)
     a, c, d = rng.uniform(0.1, 1.0, (n, nsys)), rng.uniform(0.1, 1.0, (n, nsys)), rng.standard_normal((n, nsys))
