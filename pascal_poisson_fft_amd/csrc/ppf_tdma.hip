@@ -29,7 +29,7 @@ namespace {
 // current one is solved, and a chunk's stores are younger than the loads that
 // follow it in the chain, so nothing waits for them.  One-wave workgroups
 // spread a few thousand systems over as many CUs as there are waves.  256^3
-// (many systems): 291 -> 193 us, 6.3 TB/s of the 72 bytes a row moves; cyclic
+// (many systems): 291 -> 200 us, 6.0 TB/s of the 72 bytes a row moves; cyclic
 // 6000 systems of 90 rows: 57 -> 28 us and 256 of 512 rows 363 -> 138, where a
 // row's chain of a correctly rounded division and the products that use it
 // (about 0.2 us) is what is left.
