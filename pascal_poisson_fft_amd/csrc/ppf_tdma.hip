@@ -43,8 +43,8 @@ namespace {
 // Past the last row a chunk's loads are left out: clamped to that row instead,
 // 4M systems of 3 rows took 194 us instead of 96, cyclic 309 instead of 136, 1M
 // of 20 rows 228 instead of 214.  The tests of it cost 1.3% where waves are few
-// and lines long (256^3 with its refill 304.5 us, clamped 300.7), so from 128
-// rows on, where a chunk is little of a line, loads are clamped.
+// and lines long (256^3 with its refill 304.5 us, clamped 300.7), so the plain
+// form clamps from 128 rows on, where a chunk is little of a line.
 constexpr int kTdmaThreads = 64;
 // millions of systems fill the chip whatever the workgroup's size, and its
 // launches are then fewer: 4M systems of 12 rows 492 -> 472 us (490,000 of 20
